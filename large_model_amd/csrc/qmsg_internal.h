@@ -231,6 +231,20 @@ hipError_t launch_call_reset(const Scratch &S, hipStream_t st);
 hipError_t launch_dense(const DenseArgs &a, int type, uint8_t *xqk, hipStream_t st);
 /* matmul_exact for every matrix of a call (--exact, or an F16 / Q8_0 matrix in the call). */
 hipError_t launch_dense_exact(const DenseArgs &args, int type, hipStream_t st);
+/* matmul_exact rows of one stacked expert tensor for every slot (qmsg_chain.hip): slot s's input
+ * is row slot_t[s] of x (by_token) or row s; y[s * y_stride + row]. With up (same rows, cols and
+ * type) m is the gate tensor and y takes silu(gate) * up; gu, if not NULL, [slot][2 rows] takes
+ * the gate and up rows. max_tiles bounds the slot tiles of T tokens. */
+struct ChainRows {
+    const uint8_t *w;
+    uint64_t rb, eb;
+    int type, rows, cols, by_token;
+    const float *x;
+    float *y;
+    int y_stride;
+};
+hipError_t launch_chain_rows(const char *name, const ChainRows &m, const ChainRows *up, const Scratch &S, int T,
+                             int max_tiles, float *gu, hipStream_t st);
 hipError_t launch_block_dots(const uint8_t *base, int type, uint64_t rb, uint64_t eb, int n, const int32_t *expert,
                              const int32_t *row, const int32_t *block, const Q8 *xq, int32_t *out,
                              hipStream_t st);

@@ -18,10 +18,10 @@
  * the int8 activations sit in LDS in a pair-of-blocks layout so a lane gets its two code
  * partners with one 16-byte read. */
 #include <hip/hip_runtime.h>
-#include <hip/hip_ext.h>
 
 #include <type_traits>
 
+#include "qmsg_device.h"
 #include "qmsg_internal.h"
 #include "qmsg_libm.h"
 #include "qmsg_synth.h"
@@ -53,26 +53,9 @@ extern "C" int qmsg_phase_read(void *dst, size_t bytes)
 #define PHASE(region, k) ((void)0)
 #endif
 
-/* Launch `kern` on `st`; with a timing hook installed the dispatch stamps its own events. */
-#define QLAUNCH(name, kern, grid, block, lds, st, ...)                                          \
-    do {                                                                                       \
-        hipEvent_t qa_ = nullptr, qb_ = nullptr;                                               \
-        if (qmsg::g_launch_timer)                                                              \
-            qmsg::g_launch_timer->events(qmsg::g_launch_timer->ctx, (name), &qa_, &qb_);       \
-        if (qa_)                                                                               \
-            hipExtLaunchKernelGGL(kern, (grid), (block), (lds), (st), qa_, qb_, 0u, __VA_ARGS__); \
-        else                                                                                   \
-            hipLaunchKernelGGL(kern, (grid), (block), (lds), (st), __VA_ARGS__);              \
-    } while (0)
-
 namespace qmsg {
 
 /* ------------------------------------------------------------------ scalar helpers ---- */
-
-__device__ __forceinline__ float h2f(uint32_t bits16)
-{
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
-}
 
 __device__ __forceinline__ int sdot4(int a, int b) { return __builtin_amdgcn_sdot4(a, b, 0, false); }
 
@@ -86,9 +69,6 @@ __device__ __forceinline__ float mul_f16_f32(uint32_t h, float f)
     else asm volatile("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(f));
     return r;
 }
-
-/* src/model.c:424 */
-__device__ __forceinline__ float silu_ref(float a) { return a / (1.0f + qmsg_expf(-a)); }
 
 /* An unaligned 32-bit read from LDS at an even byte address (two aligned reads). */
 __device__ __forceinline__ uint32_t lds_u32(const uint8_t *base, uint32_t a)
@@ -187,7 +167,6 @@ __device__ void quantize_block_store(const float *v, Q8 *dst, uint32_t *pair, in
 
 /* ------------------------------------------------------------------ wave primitives ---- */
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 /* LDS ordering between the lanes of one wave (its LDS operations complete in order). */
 __device__ __forceinline__ void wave_sync()
@@ -651,12 +630,6 @@ __global__ __launch_bounds__(256) void select_kernel(SelectArgs a, int do_dispat
     PHASE(0, 7);
 }
 
-__global__ __launch_bounds__(64) void dispatch_kernel(SelectArgs a)
-{
-    __shared__ int cnt[kMaxExperts], cur[kMaxExperts], tok[kMaxExperts];
-    dispatch_slots(a, a.S.sel, cnt, cur, tok);
-}
-
 /* Inclusive sum over the block's first kMaxExperts threads (4 waves); others return 0. */
 __device__ __forceinline__ int experts_scan(int v, int *wsum)
 {
@@ -780,7 +753,6 @@ struct RowAcc {
     float lo, hi, corr;
 };
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 /* The words one lane needs from a pair of Q4_0 blocks (36 bytes at W, 4-byte aligned): its
  * code dword of each block (bytes 4p..4p+3 of qs) and both scales. */
@@ -3003,12 +2975,6 @@ __device__ __forceinline__ void mx_wait_barrier()
     asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-/* Wait for this wave's LDS accesses only (DMA still in flight), then the block barrier. */
-__device__ __forceinline__ void mx_lds_barrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 #ifndef QMSG_MX_WIDE16_SLOTS
 #define QMSG_MX_WIDE16_SLOTS 8
 #endif
@@ -4214,7 +4180,7 @@ __global__ __launch_bounds__(256) void dense_any_kernel(DenseArgs a)
  * takes this int8 path for Q4_0 / Q4_1 / Q6_K rows and dot_f32 for F32 rows (src/model.c:
  * 1009-1030, src/quant.c:134-169; with n_embd % 256 == 0 its moe_group_fast gives the same
  * numbers, src/model.c:969-1006). Block (32 rows, or 16 F32 rows; active expert blockIdx.y) as
- * exact_rows_kernel; the input of slot s is row slot_t[s] of x (by_token) or row s. */
+ * chain_rows_kernel; the input of slot s is row slot_t[s] of x (by_token) or row s. */
 struct SlotAnyArgs {
     const uint8_t *w;
     uint64_t rb, eb;
@@ -4566,151 +4532,9 @@ __global__ __launch_bounds__(256) void route_exact_kernel(const float *router, c
     if (tid < 8 && e0 + tid < X) logits[(size_t)t * X + e0 + tid] = acc;
 }
 
-/* Dequantised 32-block b of a row (src/quant.c:17-93): Q4_0 (q-8)*d, Q4_1 q*d+m (fused like
- * the reference build), Q8_0 q*d, Q6_K (d*sc)*q, F16 and F32 as they are. */
-__device__ __forceinline__ void dequant_block(int type, const uint8_t *row, int b, float *w)
-{
-    /* each lane reads its own row, so every load touches another cache line per lane: words
-     * as wide as the row's alignment allows (F32 / F16 rows of 32-multiples are 16-byte
-     * aligned, Q4_1 blocks 4-byte, the others 2-byte) */
-    if (type == 0) {
-        const float4 *p = (const float4 *)(row + (size_t)b * 128);
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float4 f = p[j];
-            w[4 * j] = f.x; w[4 * j + 1] = f.y; w[4 * j + 2] = f.z; w[4 * j + 3] = f.w;
-        }
-    } else if (type == 1) {
-        const u32x4 *p = (const u32x4 *)(row + (size_t)b * 64);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const u32x4 v = p[j];
-            const uint32_t u[4] = { v.x, v.y, v.z, v.w };
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                w[8 * j + 2 * k] = h2f(u[k] & 0xffffu);
-                w[8 * j + 2 * k + 1] = h2f(u[k] >> 16);
-            }
-        }
-    } else if (type == 8) {
-        const uint16_t *p = (const uint16_t *)(row + (size_t)b * 34);
-        const float d = h2f(p[0]);
-#pragma unroll
-        for (int j = 0; j < 16; j++) {
-            const uint32_t h = p[1 + j];
-            w[2 * j] = (float)(int8_t)(h & 0xff) * d;
-            w[2 * j + 1] = (float)(int8_t)(h >> 8) * d;
-        }
-    } else if (type == 14) {
-        const uint8_t *sb = row + (size_t)(b >> 3) * 210;
-        const int h = (b & 7) >> 2, g = b & 3;
-        const uint16_t *ql = (const uint16_t *)(sb + 64 * h + 32 * (g & 1)), *qh = (const uint16_t *)(sb + 128 + 32 * h);
-        const uint32_t sc = *(const uint16_t *)(sb + 192 + 8 * h + 2 * g);
-        const float d = h2f(*(const uint16_t *)(sb + 208));
-        const float d0 = d * (float)(int8_t)(sc & 0xff);
-        const float d1 = d * (float)(int8_t)(sc >> 8);
-#pragma unroll
-        for (int l2 = 0; l2 < 16; l2++) {
-            const uint32_t lo2 = ql[l2], hi2 = qh[l2];
-#pragma unroll
-            for (int k = 0; k < 2; k++) {
-                const int l = 2 * l2 + k;
-                const int lo = (lo2 >> (8 * k)) & 0xff, hb = (hi2 >> (8 * k)) & 0xff;
-                const int q = ((g < 2 ? lo & 15 : lo >> 4) | (((hb >> (2 * g)) & 3) << 4)) - 32;
-                w[l] = (l < 16 ? d0 : d1) * (float)q;
-            }
-        }
-    } else if (type == 3) {
-        const uint32_t *p = (const uint32_t *)(row + (size_t)b * 20);
-        const uint32_t dm = p[0];
-        const float d = h2f(dm & 0xffffu), m = h2f(dm >> 16);
-#pragma unroll
-        for (int j4 = 0; j4 < 4; j4++) {
-            const uint32_t c = p[1 + j4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t q = (c >> (8 * k)) & 0xff;
-                w[4 * j4 + k] = __builtin_fmaf((float)(q & 15), d, m);
-                w[4 * j4 + k + 16] = __builtin_fmaf((float)(q >> 4), d, m);
-            }
-        }
-    } else {
-        const uint16_t *p = (const uint16_t *)(row + (size_t)b * 18);
-        const float d = h2f(p[0]);
-#pragma unroll
-        for (int j2 = 0; j2 < 8; j2++) {
-            const uint32_t c = p[1 + j2];
-#pragma unroll
-            for (int k = 0; k < 2; k++) {
-                const int q = (int)((c >> (8 * k)) & 0xff);
-                w[2 * j2 + k] = (float)((q & 15) - 8) * d;
-                w[2 * j2 + k + 16] = (float)((q >> 4) - 8) * d;
-            }
-        }
-    }
-}
-
-/* y = matmul_exact rows of each active expert's matrix for its slots: one lane per row
- * (64 rows per block, blockIdx.y = active expert), up to 4 slots per pass with their input
- * rows staged in LDS. Inputs: the slot's token row of xn (by_token) or its own row of x. */
-struct ExactArgs {
-    const uint8_t *w;
-    uint64_t rb, eb;
-    int type, rows, cols, by_token;
-    const float *x;
-    float *y;
-    int y_stride, y_off;
-    /* blockIdx.z == 1: a second matrix of the same shape and inputs (up beside gate) */
-    const uint8_t *w2;
-    uint64_t rb2, eb2;
-    int type2, y_off2;
-    Scratch S;
-};
-
-__global__ __launch_bounds__(64) void exact_rows_kernel(ExactArgs a)
-{
-    extern __shared__ __align__(16) uint8_t smem[];
-    constexpr int NT = 4;
-    if ((int)blockIdx.y >= a.S.meta[0]) return;
-    const int4 wk = a.S.work[blockIdx.y];
-    const int e = wk.x, lane = threadIdx.x, r = blockIdx.x * 64 + lane, C = a.cols;
-    float *xr = (float *)smem;                                      /* [NT][C] */
-    const bool second = blockIdx.z == 1;
-    const int type = second ? a.type2 : a.type, y_off = second ? a.y_off2 : a.y_off;
-    const uint8_t *row = (second ? a.w2 + (size_t)e * a.eb2 + (size_t)min(r, a.rows - 1) * a.rb2
-                                 : a.w + (size_t)e * a.eb + (size_t)min(r, a.rows - 1) * a.rb);
-    for (int s0 = wk.y; s0 < wk.z; s0 += NT) {
-        const int nt = min(NT, wk.z - s0);
-        __syncthreads();
-        for (int i = lane; i < nt * (C / 4); i += 64) {
-            const int n = i / (C / 4), j = i - n * (C / 4);
-            const size_t src = a.by_token ? (size_t)a.S.slot_t[s0 + n] : (size_t)(s0 + n);
-            ((float4 *)xr)[i] = ((const float4 *)(a.x + src * C))[j];
-        }
-        __syncthreads();
-        float acc[NT] = { 0.0f, 0.0f, 0.0f, 0.0f };
-        for (int b = 0; b < C / 32; b++) {
-            float w[32];
-            dequant_block(type, row, b, w);
-#pragma unroll
-            for (int n = 0; n < NT; n++)
-                if (n < nt)
-#pragma unroll
-                    for (int j = 0; j < 32; j++) acc[n] = __builtin_fmaf(w[j], xr[n * C + 32 * b + j], acc[n]);
-        }
-        if (r < a.rows)
-            for (int n = 0; n < nt; n++) a.y[(size_t)(s0 + n) * a.y_stride + y_off + r] = acc[n];
-    }
-}
-
 hipError_t launch_layer_slots(const Shape &s, const LayerDev &L, const Scratch &S, const float *xn, float *out, int T,
                               int exact, int debug, hipStream_t st, int down_only)
 {
-    SelectArgs sa;
-    sa.X = s.X;
-    sa.K = s.K;
-    sa.T = T;
-    sa.S = S;
     if (down_only) {
         /* routing, gate/up and SwiGLU done by the integer kernels */
     } else if (exact) {
@@ -4723,53 +4547,41 @@ hipError_t launch_layer_slots(const Shape &s, const LayerDev &L, const Scratch &
         if (e != hipSuccess) return e;
     }
     if (!down_only) {
-        QLAUNCH("select", select_kernel, dim3(T), dim3(256), 0, st, sa, 0);
-        QLAUNCH("dispatch", dispatch_kernel, dim3(1), dim3(64), 0, st, sa);
+        const hipError_t e = launch_select(s, S, T, 0, st);
+        if (e != hipSuccess) return e;
     }
     const int maxact = s.X < T * s.K ? s.X : T * s.K;
-    const struct { const uint8_t *w; uint64_t rb, eb; int type, rows, cols, by_token; const float *x; float *y;
-                   int stride, off; } m[3] = {
-        { L.gate, L.gate_rb, L.gate_eb, L.gate_type, s.F, s.E, 1, xn, S.gu, 2 * s.F, 0 },
-        { L.up, L.up_rb, L.up_eb, L.up_type, s.F, s.E, 1, xn, S.gu, 2 * s.F, s.F },
-        { L.down, L.down_rb, L.down_eb, L.down_type, s.E, s.F, 0, S.act, S.dn, s.E, 0 },
+    const int max_tiles = maxact + T * s.K / kTileN + 1;
+    const ChainRows m[3] = {
+        { L.gate, L.gate_rb, L.gate_eb, L.gate_type, s.F, s.E, 1, xn, S.gu, 2 * s.F },
+        { L.up, L.up_rb, L.up_eb, L.up_type, s.F, s.E, 1, xn, S.gu + s.F, 2 * s.F },
+        { L.down, L.down_rb, L.down_eb, L.down_type, s.E, s.F, 0, S.act, S.dn, s.E },
     };
+    /* --exact, and F16 / Q8_0 rows at any setting (outside qms_fast_supported, so the
+     * reference's qms_matmul takes matmul_exact for them): the fp32 chain */
+    auto chain_rows = [&](int t) { return exact || t == 1 || t == 8; };
+    bool act_done = down_only != 0;
     for (int i = down_only ? 2 : 0; i < 3; i++) {
-        if (i == 2 && !down_only) {
+        if (i == 2 && !act_done) {
             const int n = T * s.K * s.F;
             QLAUNCH("swiglu", swiglu_kernel, dim3((n + 255) / 256), dim3(256), 0, st, S, s.F, T * s.K);
         }
         const char *name = i == 2 ? "down" : "gateup";
-        /* --exact, and F16 / Q8_0 rows at any setting (outside qms_fast_supported, so the
-         * reference's qms_matmul takes matmul_exact for them): the fp32 chain */
-        auto chain_rows = [&](int t) { return exact || t == 1 || t == 8; };
-        /* gate and up in one launch (grid z = 2) when they take the same kernel */
-        const bool pair = i == 0 && (chain_rows(m[0].type) ? chain_rows(m[1].type)
-                                                           : !chain_rows(m[1].type) && m[1].type == m[0].type);
+        /* gate and up of one type in one launch */
+        const bool pair = i == 0 && m[1].type == m[0].type;
         if (chain_rows(m[i].type)) {
-            ExactArgs a;
-            a.S = S;
-            a.w = m[i].w;
-            a.rb = m[i].rb;
-            a.eb = m[i].eb;
-            a.type = m[i].type;
-            a.rows = m[i].rows;
-            a.cols = m[i].cols;
-            a.by_token = m[i].by_token;
-            a.x = m[i].x;
-            a.y = m[i].y;
-            a.y_stride = m[i].stride;
-            a.y_off = m[i].off;
-            a.w2 = m[1].w;
-            a.rb2 = m[1].rb;
-            a.eb2 = m[1].eb;
-            a.type2 = m[1].type;
-            a.y_off2 = m[1].off;
-            /* input rows for the slots of one pass: at most min(4, T), an expert's slots
-             * being distinct tokens */
-            const size_t lds = (size_t)min(4, T) * m[i].cols * 4;
-            if (lds > 160 * 1024) return hipErrorInvalidValue;
-            QLAUNCH(name, exact_rows_kernel, dim3((m[i].rows + 63) / 64, maxact, pair ? 2 : 1), dim3(64), lds, st, a);
-            if (pair) i++;
+            /* the widths this path takes: four input rows (or the batch's) in 160 KiB */
+            if ((size_t)min(4, T) * m[i].cols * 4 > 160 * 1024) return hipErrorInvalidValue;
+            ChainRows r = m[i];
+            if (pair) {
+                r.y = S.act;
+                r.y_stride = s.F;
+                act_done = true;
+                i++;
+            }
+            const hipError_t e = launch_chain_rows(name, r, pair ? &m[1] : nullptr, S, T, max_tiles,
+                                                   pair && debug ? S.gu : nullptr, st);
+            if (e != hipSuccess) return e;
             continue;
         }
         SlotAnyArgs a;
@@ -4782,12 +4594,12 @@ hipError_t launch_layer_slots(const Shape &s, const LayerDev &L, const Scratch &
         a.by_token = m[i].by_token;
         a.x = m[i].x;
         a.y = m[i].y;
-        a.y_stride = m[i].stride;
-        a.y_off = m[i].off;
+        a.y_stride = m[i].y_stride;
+        a.y_off = 0;
         a.w2 = m[1].w;
         a.rb2 = m[1].rb;
         a.eb2 = m[1].eb;
-        a.y_off2 = m[1].off;
+        a.y_off2 = s.F;
         const int nb = m[i].cols / 32, NT = dense_any_nt(m[i].type, T, nb);
         if (!NT) return hipErrorInvalidValue;
         const size_t lds = m[i].type == 0 ? 0 : (size_t)NT * nb * kDenseAnyRec;
@@ -4818,68 +4630,6 @@ hipError_t launch_layer_slots(const Shape &s, const LayerDev &L, const Scratch &
         QLAUNCH("combine", combine_kernel, dim3(n / (4 * combine_threads(s.E))), dim3(combine_threads(s.E)), 0, st, S,
                 s.E, s.K, T, out);
     else QLAUNCH("combine", combine_any_kernel, dim3((n + 255) / 256), dim3(256), 0, st, S, s.E, s.K, T, out);
-    return hipGetLastError();
-}
-
-/* ------------------------------------------------------------------ dense rows, fp32 chains ---- */
-
-/* qms_matmul_n's matmul_exact (src/quant.c:97-115) for calls the fast loop does not take: the
- * --exact mode, or any matrix of a type outside qms_fast_supported (F16, Q8_0) in the call,
- * which sends every matrix of it there (src/quant.c:131-141). One lane per row of the call's
- * matrices (one type per launch), its dequantised 32-blocks against up to NT tokens staged in
- * LDS, acc = fma(w, x, acc) in element order. Rows past a matrix's end read its last row and
- * store nothing. */
-template <int NT>
-__global__ __launch_bounds__(64) void dense_exact_kernel(DenseArgs a, int type)
-{
-    extern __shared__ __align__(16) uint8_t smem[];
-    float *xr = (float *)smem;                        /* [NT][C] */
-    int mi = 0;
-#pragma unroll
-    for (int i = 1; i < kDenseMats; i++)
-        if (i < a.nm && (int)blockIdx.x >= a.m[i].first_block) mi = i;
-    const DenseMat M = a.m[mi];
-    const int lane = threadIdx.x, C = a.C;
-    const int row = ((int)blockIdx.x - M.first_block) * 64 + lane;
-    const uint8_t *wr = M.w + (size_t)min(row, M.rows - 1) * a.rb;
-    for (int t0 = 0; t0 < a.T; t0 += NT) {
-        const int nt = min(NT, a.T - t0);
-        __syncthreads();
-        for (int i = lane; i < nt * (C / 4); i += 64)
-            ((float4 *)xr)[i] = ((const float4 *)(a.x + (size_t)t0 * C))[i];
-        __syncthreads();
-        float acc[NT];
-#pragma unroll
-        for (int n = 0; n < NT; n++) acc[n] = 0.0f;
-        for (int b = 0; b < C / 32; b++) {
-            float w[32];
-            dequant_block(type, wr, b, w);
-#pragma unroll
-            for (int n = 0; n < NT; n++)
-                if (n < nt)
-#pragma unroll
-                    for (int j = 0; j < 32; j++) acc[n] = __builtin_fmaf(w[j], xr[n * C + 32 * b + j], acc[n]);
-        }
-        if (row < M.rows)
-            for (int n = 0; n < nt; n++) M.y[(size_t)(t0 + n) * M.rows + row] = acc[n];
-    }
-}
-
-hipError_t launch_dense_exact(const DenseArgs &args, int type, hipStream_t st)
-{
-    DenseArgs a = args;
-    const size_t row_lds = (size_t)a.C * 4;
-    const int NT = 4 * row_lds <= 160 * 1024 ? 4 : (2 * row_lds <= 160 * 1024 ? 2 : 1);
-    if (row_lds > 160 * 1024) return hipErrorInvalidValue;
-    int nblk = 0;
-    for (int i = 0; i < a.nm; i++) {
-        a.m[i].first_block = nblk;
-        nblk += (a.m[i].rows + 63) / 64;
-    }
-    const size_t lds = NT * row_lds;
-    if (NT == 4) QLAUNCH("dense", dense_exact_kernel<4>, dim3(nblk), dim3(64), lds, st, a, type);
-    else if (NT == 2) QLAUNCH("dense", dense_exact_kernel<2>, dim3(nblk), dim3(64), lds, st, a, type);
-    else QLAUNCH("dense", dense_exact_kernel<1>, dim3(nblk), dim3(64), lds, st, a, type);
     return hipGetLastError();
 }
 
