@@ -721,6 +721,14 @@ int qmsg_gguf_upload_mat(qmsg_ctx *c, const qmsg_gguf *g, const char *name, int 
     return QMSG_OK;
 }
 
+/* Every layer and dense call gets an epoch of its own: record producers store it in a flag word
+ * when a record falls outside the MFMA kernels' scaled range, and the consumers compare. */
+static uint64_t next_epoch()
+{
+    static std::atomic<uint64_t> epochs{ 0 };
+    return ++epochs;
+}
+
 /* Device buffer *p of at least `bytes`, reallocated (after the stream drains) when smaller. */
 static int grow(qmsg_ctx *c, void **p, size_t *cap, size_t bytes)
 {
@@ -750,8 +758,8 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
     if (T == 0) return QMSG_OK;
     if (!d_x || ((uintptr_t)d_x & 15)) return fail(c, QMSG_E_INVALID, "qmsg_matmul_n: x must be 16-byte aligned");
     HIP_TRY(c, hipSetDevice(c->device));
-    if (T >= kDenseQuantT) {
-        const int rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, (size_t)T * (size_t)(C / 64) * kPairBytes);
+    if (T >= kDenseRecordT) {
+        const int rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, dense_record_bytes((size_t)T, (size_t)C));
         if (rc) return rc;
     }
     /* qms_matmul_n's choice for the whole call (src/quant.c:131-141): the fast loop, or
@@ -783,7 +791,7 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
             done[(size_t)j] = true;
         }
         if (exact) LAUNCH(c, "dense", launch_dense_exact(a, type, c->stream));
-        else LAUNCH(c, "dense", launch_dense(a, type, (uint8_t *)c->dense_xqk, c->stream));
+        else LAUNCH(c, "dense", launch_dense(a, type, (uint8_t *)c->dense_xqk, next_epoch(), c->stream));
     }
     return QMSG_OK;
 }
@@ -825,11 +833,8 @@ int qmsg_matmul_n(qmsg_ctx *c, const int *ids, int nW, const float *x, int T, fl
 static int run_layer_s(qmsg_ctx *c, const Scratch &S0, int layer, const float *d_xn, int T, float *d_out, int debug,
                        const NormIn *ni = nullptr)
 {
-    /* every layer call gets an epoch of its own: record producers store it in S.mxflag when a
-     * record falls outside the MFMA kernels' scaled range, and the consumers compare */
-    static std::atomic<uint64_t> epochs{ 0 };
     Scratch S = S0;
-    S.epoch = ++epochs;
+    S.epoch = next_epoch();
     int rc = check_layer_index(c, layer);
     if (rc) return rc;
     const LayerStore &L = c->layers[(size_t)layer];

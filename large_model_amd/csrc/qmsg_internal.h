@@ -134,6 +134,8 @@ struct DenseArgs {
 /* Batches of at least this many rows are quantised once by a separate launch; smaller ones
  * inside every dense block. */
 constexpr int kDenseQuantT = 8;
+/* Batches from which a dense call may need the record buffer (its MFMA kernels: from 5 rows). */
+constexpr int kDenseRecordT = 5;
 
 /* Launchers (qmsg_kernels.hip). Each returns hipSuccess or the launch error. */
 hipError_t launch_route(const Shape &s, const LayerDev &L, const Scratch &S, const float *xn, int T,
@@ -226,9 +228,11 @@ hipError_t launch_exp(const double *x, int n, double *out, hipStream_t st);
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
 /* p[0 .. n-1] = v (a kernel, not a memset node: safe inside a captured graph). */
 hipError_t launch_call_reset(const Scratch &S, hipStream_t st);
-/* The dense rows kernel; for T >= kDenseQuantT the input records are formed first into xqk
- * (T*C/64 records of 96 bytes). */
-hipError_t launch_dense(const DenseArgs &a, int type, uint8_t *xqk, hipStream_t st);
+/* The dense rows kernel; for T >= kDenseQuantT (MFMA kernels: kDenseRecordT) the input records are formed first into xqk
+ * (dense_record_bytes), whose flag word takes epoch (unique per call) when one is outside the
+ * MFMA kernels' scaled range. */
+inline size_t dense_record_bytes(size_t T, size_t C) { return 256 + T * (C / 32) * kMxRec; }
+hipError_t launch_dense(const DenseArgs &a, int type, uint8_t *xqk, uint64_t epoch, hipStream_t st);
 /* matmul_exact for every matrix of a call (--exact, or an F16 / Q8_0 matrix in the call). */
 hipError_t launch_dense_exact(const DenseArgs &args, int type, hipStream_t st);
 /* matmul_exact rows of one stacked expert tensor for every slot (qmsg_chain.hip): slot s's input

@@ -2424,6 +2424,7 @@ struct MxArgs {
     uint8_t *rec_out;            /* gate/up: the activation records [slot][F/32] */
     int rec_out_hi16;            /* gate/up: the down rows are Q4_0 / Q4_1 (records' lanes 4-7 x / 16) */
     Scratch S;
+    DenseArgs d;                 /* dense rows: the matrices, T and C (rec: [token][C/32])      */
 };
 
 /* LDS bytes of one staged weight row (kMxC blocks): Q4_0 144, Q4_1 160, Q6_K one super-block
@@ -2873,7 +2874,7 @@ __device__ __forceinline__ void mx_chunk_q6(const uint8_t *W, const uint8_t *R, 
 /* One Q6_K block B of the staged chunk on the 16x16x16 instructions (the layout of mx_block16):
  * half h of the 32-block is sub-block 2g + h, so each instruction's lane sums share one
  * sub-scale per row; one d_w d_x product and one half-sum offset step per (tile, quad, block). */
-template <int NQ, int O, int B, int TS>
+template <int NQ, int O, int B, int NT, int TS>
 __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[2][kMxNA], float (&cr)[2][4])
 {
     constexpr int RS = mx_rstride(14), RB = B * mx_recl(14);
@@ -2881,7 +2882,7 @@ __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[
     f16x4 b[2][2];
     float sc[2][2];
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
+    for (int t = 0; t < NT; t++) {
         w[t] = mx_weights_q6<O, B, TS>(st.q, st.dw, t, 0);
         b[t][0] = __builtin_shufflevector(w[t].op, w[t].op, 0, 1, 2, 3);
         b[t][1] = __builtin_shufflevector(w[t].op, w[t].op, 4, 5, 6, 7);
@@ -2901,7 +2902,7 @@ __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[
         }
         const f16x4 aop = __builtin_bit_cast(f16x4, av);
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int t = 0; t < NT; t++)
             S[k][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(aop, b[t][h], f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }, 0, 0, 0);
     };
     issue(0, 0);
@@ -2911,16 +2912,16 @@ __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[
         if (u + 1 < 2 * NQ) issue(u + 1, k ^ 1);
         if (h == 0) {
 #pragma unroll
-            for (int t = 0; t < 2; t++) dd[t] = mix_mul(w[t].dw, xd[q]);
+            for (int t = 0; t < NT; t++) dd[t] = mix_mul(w[t].dw, xd[q]);
         }
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int t = 0; t < NT; t++)
 #pragma unroll
             for (int v = 0; v < 4; v++)
                 acc[t][2 * q + h][v] = __builtin_fmaf(S[k][t][v] * sc[t][h], dd[t], acc[t][2 * q + h][v]);
         if (h == 1) {
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < NT; t++) {
                 /* sc[2g]*s16[0] + sc[2g+1]*s16[1] in one packed int16 dot */
                 const int ssum = sdot2_i16(w[t].sab, s16p[q]);
                 cr[t][q] = __builtin_fmaf(dd[t], (float)ssum, cr[t][q]);
@@ -2930,7 +2931,7 @@ __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[
 }
 
 /* A staged Q6_K super-block on the 16x16x16 instructions, its 8 blocks unrolled. */
-template <int NQ, int O, int TS>
+template <int NQ, int O, int NT, int TS>
 __device__ __forceinline__ void mx_chunk16_q6(const uint8_t *W, const uint8_t *R, int lr, int lg, int offa_lo,
                                               int offa_hi, f32x4 (&acc)[2][kMxNA], float (&cr)[2][4])
 {
@@ -2942,21 +2943,21 @@ __device__ __forceinline__ void mx_chunk16_q6(const uint8_t *W, const uint8_t *R
     st.q = (LdsPtr)(W + lr * WS + 4 * lg);
     st.dw = (LdsPtr)(W + lr * WS);
     mx_opaque(st);
-    mx_block16_q6<NQ, O, 0, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 0, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
-    mx_block16_q6<NQ, O, 1, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 1, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
-    mx_block16_q6<NQ, O, 2, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 2, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
-    mx_block16_q6<NQ, O, 3, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 3, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
-    mx_block16_q6<NQ, O, 4, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 4, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
-    mx_block16_q6<NQ, O, 5, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 5, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
-    mx_block16_q6<NQ, O, 6, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 6, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
-    mx_block16_q6<NQ, O, 7, TS>(st, acc, cr);
+    mx_block16_q6<NQ, O, 7, NT, TS>(st, acc, cr);
 }
 
 /* The LDS DMA: `bytes` (4 or 16) from src of every active lane to dst + lane * bytes. */
@@ -3013,19 +3014,22 @@ constexpr int mx_waves()
     return NB == 1 ? 4 : (160 * 1024 / mx_lds_bytes(TYPE, WSG, PPW, NW, NB, NT)) * NW / 4 >= 6 ? 6 : 4;
 }
 
-/* Gate/up (GU = 1: gate rows against the token's input records, the same up rows, SwiGLU, the
- * int8 activation blocks and their records) or down (GU = 0: dn rows) of one slot tile, with NB
+/* Gate/up (MODE 1: gate rows against the token's input records, the same up rows, SwiGLU, the
+ * int8 activation blocks and their records) or down (MODE 0: dn rows) of one slot tile, or the rows
+ * of a dense product (MODE 2: the matrix whose block range holds blockIdx.x, every token a slot,
+ * the last block of a matrix moved up to whole rows and storing only those past the one before), with NB
  * staging buffers: 2 (the next chunk's copy in flight while this one computes) or 1 (copy, wait,
  * compute; the other blocks on the CU hide the copy). Several blocks share a CU, which hides the
  * LDS and memory latency. */
-template <int TYPE, int WSG, int GU, int PPW, int NW, int NB, int NT>
+template <int TYPE, int WSG, int MODE, int PPW, int NW, int NB, int NT>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(mx_waves<TYPE, WSG, PPW, NW, NB, NT>(),
                                                                          mx_waves<TYPE, WSG, PPW, NW, NB, NT>())))
 void mx_kernel(MxArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem[];
     using Lay = MxLayout<TYPE, WSG, PPW, NW, NT>;
-    static_assert(NT == 2 || (NT == 1 && TYPE != 14), "one-tile waves take Q4_0 / Q4_1 rows");
+    constexpr bool GU = MODE == 1, DENSE = MODE == 2;
+    static_assert(NT == 2 || (NT == 1 && !(GU && TYPE == 14)), "Q6_K gate/up steps two-tile rows");
     /* Q6_K gate/up (4-byte DMA units) steps through its gate rows, then its up rows */
     constexpr bool QS6 = GU && TYPE == 14;
     /* gate/up on two-tile waves: the RWG/2 gate rows staged first, then the same up rows, so
@@ -3041,21 +3045,35 @@ void mx_kernel(MxArgs a)
 #endif
     constexpr int RWG = Lay::RWG, SWG = Lay::SWG, WS = Lay::WS, BUF = Lay::BUF;
     static_assert(PPW <= 4 || X16Q, "waves of more than 8 slots take the 16x16x16 quads");
-    if ((int)blockIdx.y >= a.S.meta[1]) return;
-    const int4 tl = a.S.tiles[blockIdx.y];
-    const int e = tl.x, s0 = tl.y + (int)blockIdx.z * SWG, ns = min(SWG, tl.z - s0);
-    if (ns <= 0) return;
+    int e = 0, s0, ns, R0 = (int)blockIdx.x * (GU ? RWG / 2 : RWG), skip = 0, mi = 0;
+    if constexpr (DENSE) {
+#pragma unroll
+        for (int i = 1; i < kDenseMats; i++)
+            if (i < a.d.nm && (int)blockIdx.x >= a.d.m[i].first_block) mi = i;
+        const int r = ((int)blockIdx.x - a.d.m[mi].first_block) * RWG;
+        R0 = min(r, a.d.m[mi].rows - RWG);
+        skip = r - R0;
+        s0 = (int)blockIdx.y * SWG;
+        ns = min(SWG, a.d.T - s0);
+    } else {
+        if ((int)blockIdx.y >= a.S.meta[1]) return;
+        const int4 tl = a.S.tiles[blockIdx.y];
+        e = tl.x;
+        s0 = tl.y + (int)blockIdx.z * SWG;
+        ns = min(SWG, tl.z - s0);
+        if (ns <= 0) return;
+    }
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);          /* wave-uniform */
     const int wr = wave / WSG, ws = wave % WSG, kh = lg & 1, jd = lg >> 1;
-    const int nb = (GU ? a.E : a.F) >> 5, nch = nb / kMxC;
-    const int R0 = (int)blockIdx.x * (GU ? RWG / 2 : RWG);
+    const int nb = (DENSE ? a.d.C : (GU ? a.E : a.F)) >> 5, nch = nb / kMxC;
 
     /* row i of the staged tile: for gate/up on two-tile waves gate row R0 + i below RWG/2 and
      * up row R0 + i - RWG/2 above; on one-tile waves row group g = i / 32 holds gate rows
      * R0 + 16g .. R0 + 16g + 15 and then the same up rows. Byte offsets inside one expert's
      * matrix fit 31 bits (mx_supported); the expert bases are wave-uniform. */
-    const uint8_t *wb0 = a.w0 + (size_t)e * a.eb, *wb1 = GU ? a.w1 + (size_t)e * a.eb : wb0;
+    const uint8_t *wb0 = DENSE ? a.d.m[mi].w + (size_t)R0 * a.rb : a.w0 + (size_t)e * a.eb;
+    const uint8_t *wb1 = GU ? a.w1 + (size_t)e * a.eb : wb0;
     const uint32_t rb = (uint32_t)a.rb;
     /* slot i's records (slots past the tile repeat its last slot) */
     auto rec_ptr = [&](int i) -> const uint8_t * {
@@ -3084,7 +3102,7 @@ void mx_kernel(MxArgs a)
         *u_out = u;
         /* two-tile gate/up: gate rows first, up rows from staged row RWG/2 on (GSEP); one-tile
          * gate/up: 16 gate rows, then the same up rows (bit 31 of the offset: an up row) */
-        const int row = GSEP ? R0 + (i % (RWG / 2)) : (GU ? R0 + 16 * (i >> 5) + (i & 15) : R0 + i);
+        const int row = GSEP ? R0 + (i % (RWG / 2)) : (GU ? R0 + 16 * (i >> 5) + (i & 15) : (DENSE ? i : R0 + i));
         const uint32_t up = GU && !GSEP && (i & 31) >= 16 ? 0x80000000u : 0u;
         return ((uint32_t)row * rb + (uint32_t)(Lay::WUNIT * u)) | up;
     };
@@ -3181,6 +3199,12 @@ void mx_kernel(MxArgs a)
      * issues its share of the DMA and meets every barrier, whatever its NP (0 included). */
     constexpr float scale = finish_scale(TYPE);
     float *res = (float *)smem;                                   /* [RWG][SWG + 1], after the loop */
+    auto put = [&](int row, int sl, float val) {
+        if constexpr (GU) res[row * (SWG + 1) + sl] = val;
+        else if constexpr (DENSE) {
+            if (sl < ns && row >= skip) a.d.m[mi].y[(size_t)(s0 + sl) * a.d.m[mi].rows + R0 + row] = val;
+        } else if (sl < ns) a.S.dn[(size_t)(s0 + sl) * a.E + R0 + row] = val;
+    };
     auto run = [&](auto npc, auto scc, auto x16c) {
         constexpr int NP = decltype(npc)::value;
         constexpr bool SC = decltype(scc)::value;
@@ -3225,8 +3249,8 @@ void mx_kernel(MxArgs a)
                 const uint8_t *Rl = (NB == 3 ? rarea : smem + buf * BUF + Lay::WBYTES) + (2 * PPW * ws) * Lay::RS;
                 if constexpr (TYPE == 14 && X16) {
                     constexpr int TS6 = QS6 ? RWG / 2 : 16;
-                    if (c & 1) mx_chunk16_q6<NP / 2, 2, TS6>(Wl, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
-                    else mx_chunk16_q6<NP / 2, 0, TS6>(Wl, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
+                    if (c & 1) mx_chunk16_q6<NP / 2, 2, NT, TS6>(Wl, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
+                    else mx_chunk16_q6<NP / 2, 0, NT, TS6>(Wl, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
                 } else if constexpr (TYPE == 14) {
                     constexpr int TS6 = QS6 ? RWG / 2 : 16;
                     if (c & 1) mx_chunk_q6<NP, 2, TS6>(Wl, Rl, lr, lg, kh, jd, offa_lo, offa_hi, acc, cr);
@@ -3257,8 +3281,7 @@ void mx_kernel(MxArgs a)
                     const float h = ((lo[0] + hi[0]) + (lo[2] + hi[2])) + ((lo[1] + hi[1]) + (lo[3] + hi[3]));
                     const float val = h - scale * cr[t][q];
                     const int row = 16 * NT * wr + 16 * t + lr, sl = 2 * PPW * ws + 4 * q + lg;
-                    if (GU) res[row * (SWG + 1) + sl] = val;
-                    else if (sl < ns) a.S.dn[(size_t)(s0 + sl) * a.E + R0 + row] = val;
+                    put(row, sl, val);
                 }
             return;
         }
@@ -3282,8 +3305,7 @@ void mx_kernel(MxArgs a)
                     const float h = ((q[0] + o[0]) + (q[2] + o[2])) + ((q[1] + o[1]) + (q[3] + o[3]));
                     const float val = h - scale * crv;
                     const int row = 32 * wr + 16 * t + lr, sl = 2 * PPW * ws + 2 * p + jd;
-                    if (GU) res[row * (SWG + 1) + sl] = val;
-                    else if (sl < ns) a.S.dn[(size_t)(s0 + sl) * a.E + R0 + row] = val;
+                    put(row, sl, val);
                 }
             }
     };
@@ -3314,7 +3336,7 @@ void mx_kernel(MxArgs a)
     if constexpr (TYPE == 14) by_pairs(std::true_type{});
     else if (a.S.mxflag[GU ? 0 : 1] != a.S.epoch) by_pairs(std::true_type{});
     else by_pairs(std::false_type{});
-    if (!GU) return;
+    if constexpr (!GU) return;
     __syncthreads();
     /* a = silu(g) * u (src/model.c:989-994) into the gate rows of res, then the int8 blocks of
      * whole 32-row blocks (src/model.c:996-997) and their records. F-row fr sits in row group
@@ -3335,7 +3357,7 @@ void mx_kernel(MxArgs a)
         }
     }
     __syncthreads();
-    constexpr int NFB = RWG / 64;                                  /* activation blocks per slot */
+    constexpr int NFB = GU ? RWG / 64 : 1;                                  /* activation blocks per slot */
     for (int i = tid; i < SWG * NFB; i += 64 * NW) {
         const int sl = i / NFB, g = i - sl * NFB;
         if (sl >= ns) continue;
@@ -3404,6 +3426,17 @@ static void launch_mx_shape(const MxArgs &a, int rows, int maxt, hipStream_t st)
 {
     using Lay = MxLayout<TYPE, WSG, PPW, NW, NT>;
     const size_t lds = (size_t)mx_lds_bytes(TYPE, WSG, PPW, NW, NB, NT);
+    if constexpr (GU == 2) {
+        MxArgs b = a;
+        int nblk = 0;
+        for (int i = 0; i < b.d.nm; i++) {
+            b.d.m[i].first_block = nblk;
+            nblk += (b.d.m[i].rows + Lay::RWG - 1) / Lay::RWG;
+        }
+        QLAUNCH("dense", (mx_kernel<TYPE, WSG, GU, PPW, NW, NB, NT>), dim3(nblk, (b.d.T + Lay::SWG - 1) / Lay::SWG),
+                dim3(64 * NW), lds, st, b);
+        return;
+    }
     QLAUNCH(GU ? "gateup" : "down", (mx_kernel<TYPE, WSG, GU, PPW, NW, NB, NT>),
             dim3(rows / (GU ? Lay::RWG / 2 : Lay::RWG), maxt, kTileN / Lay::SWG), dim3(64 * NW), lds, st, a);
 }
@@ -3542,6 +3575,83 @@ __global__ void dense_quant_kernel(const float *x, int C, int T, uint8_t *xqk)
         v[4 * j] = f.x; v[4 * j + 1] = f.y; v[4 * j + 2] = f.z; v[4 * j + 3] = f.w;
     }
     store_pair_half(quantize_block(v), (uint32_t *)(xqk + ((size_t)t * (nb >> 1) + (blk >> 1)) * kPairBytes), blk & 1);
+}
+
+/* The same rows' MFMA records (T * C / 32 of kMxRec bytes). */
+__global__ void dense_mx_quant_kernel(const float *x, int n, uint8_t *rec, uint64_t *flag, uint64_t epoch, int hi16)
+{
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= n) return;
+    float v[32];
+    const float4 *src = (const float4 *)(x + (size_t)b * 32);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float4 f = src[j];
+        v[4 * j] = f.x; v[4 * j + 1] = f.y; v[4 * j + 2] = f.z; v[4 * j + 3] = f.w;
+    }
+    if (!mx_store_record(quantize_block(v), rec + (size_t)b * kMxRec, hi16)) *flag = epoch;
+}
+
+/* Dense rows on the MFMA kernels (mx_kernel MODE 2). Most dense grids are small (72 blocks of 128
+ * rows for q/k/v at the 235B shape), so waves take one 16-row tile and blocks 64 rows: twice the
+ * waves, each with half the chain work between its waits. us per trunk layer (two launches and
+ * their records' two, 8.5-15 more), one-tile / the expert kernels' two-tile blocks:
+ *   235B Q4_0, 64 x 4 slots: 51 / 70 at 8 tokens, 64 / 82 at 32, 104 / 111 at 64;
+ *   64 x 16 (8 waves): 150 / 164 at 128, 274 / 269 at 256, 531 / 489 at 512, where the grid is
+ *   large enough for 128 x 16-slot two-tile waves, which unpack each row tile once;
+ *   235B Q6_K, 64 x 4: 105 / 187 at 8, 156 / 247 at 32; 64 x 8: 200 / 310 at 64; 64 x 16
+ *   (8 waves): 285 / 406 at 128; 64 x 16 (4 waves of 16 slots): 496 / 602 at 256, 935 / 1104 at 512.
+ * The token-parallel row kernels they replace: Q4_0 126 at 16 tokens, 474 at 64, 3800 at 512; Q6_K
+ * 247, 930. */
+template <int TYPE>
+static void launch_dense_mx_type(const MxArgs &a, hipStream_t st)
+{
+    long rows = 0;
+    for (int i = 0; i < a.d.nm; i++) rows += a.d.m[i].rows;
+    const long blocks = rows / 64 * ((a.d.T + 15) / 16);             /* of 64 rows x 16 tokens */
+    if constexpr (TYPE == 14) {
+        if (a.d.T <= 32) launch_mx_shape<14, 2, 1, 2, 4, 2, 1>(a, 0, 0, st);
+        else if (a.d.T < 96) launch_mx_shape<14, 2, 1, 4, 4, 2, 1>(a, 0, 0, st);
+        else if (blocks < 2048) launch_mx_shape<14, 2, 2, 4, 8, 2, 1>(a, 0, 0, st);
+        else launch_mx_shape<14, 2, 1, 8, 4, 1, 1>(a, 0, 0, st);
+    } else {
+        if (a.d.T <= 64) launch_mx_shape<TYPE, 2, 1, 2, 4, 2, 1>(a, 0, 0, st);
+        else if (blocks < 1536) launch_mx_shape<TYPE, 2, 2, 4, 8, 2, 1>(a, 0, 0, st);
+        else launch_mx_shape<TYPE, 2, 1, 8, 4, 3>(a, 0, 0, st);
+    }
+}
+
+/* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
+ * read (Q6_K: 4-byte aligned), a block's rows in each matrix, and enough tokens. us per launch
+ * pair with the records at the 235B / 30B shapes, MFMA / row kernels: Q4_0 58 / 43 and 35 / 21 at
+ * 4 tokens, about 59 / 72 and 35 / 33 at 6, 63 / 134 at 16; Q6_K 108 / 85 and 59 / 36 at 4, 112 /
+ * 137 and 60 / 49 at 6, 64 / 109 (30B) at 16, where the row kernels take another pass. */
+static bool dense_mx_takes(const DenseArgs &a, int type)
+{
+    if ((type != 2 && type != 3 && type != 14) || a.C % 256 || (type == 14 && a.rb % 4) || a.T > 4 * 65535) return false;
+    long rows = 0;
+    for (int i = 0; i < a.nm; i++) {
+        if (a.m[i].rows < 128) return false;
+        rows += a.m[i].rows;
+    }
+    return a.T > 8 || (a.T > 4 && rows * a.C >= 1l << 24);
+}
+
+static hipError_t launch_dense_mx(const DenseArgs &d, int type, uint8_t *buf, uint64_t epoch, hipStream_t st)
+{
+    const int n = d.T * (d.C / 32);
+    MxArgs a{};
+    a.d = d;
+    a.rb = d.rb;
+    a.rec = buf + 256;
+    a.S.mxflag = (uint64_t *)buf;
+    a.S.epoch = epoch;
+    QLAUNCH("dquant", dense_mx_quant_kernel, dim3((n + 255) / 256), dim3(256), 0, st, d.x, n, buf + 256,
+            a.S.mxflag + 1, epoch, type != 14 ? 1 : 0);
+    if (type == 14) launch_dense_mx_type<14>(a, st);
+    else if (type == 3) launch_dense_mx_type<3>(a, st);
+    else launch_dense_mx_type<2>(a, st);
+    return hipGetLastError();
 }
 
 /* qms_matmul_n's fast loop (src/quant.c:151-169) over up to kDenseMats matrices of one type
@@ -4314,10 +4424,11 @@ hipError_t launch_f32_rows(const float *w, int rows, int C, const float *x, int 
     return hipGetLastError();
 }
 
-hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, hipStream_t st)
+hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t epoch, hipStream_t st)
 {
     DenseArgs a = args;
     const int nb = a.C / 32;
+    if (xqk && dense_mx_takes(a, type)) return launch_dense_mx(a, type, xqk, epoch, st);
     if (type != 0 && (type == 14 ? nb % 64 != 0 : nb % 8 != 0)) {
         /* widths the chunked kernels do not take: one direct-read pass per NT tokens */
         const int NT = dense_any_nt(type, a.T, nb);
