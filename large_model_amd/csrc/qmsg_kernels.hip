@@ -2568,6 +2568,7 @@ __device__ __forceinline__ float mix_fma_hi(uint32_t h, float f, float c)
  * trip covers two blocks; the second block and the pairs and tiles are immediate offsets. */
 struct MxStreams {
     LdsPtr alo, ahi, d, q, dw;
+    uint32_t sh;                 /* Q6_K rows of alternating alignment: q6_word's shift */
 };
 
 /* The empty asm keeps each stream a single register: otherwise every (pair, stream) address
@@ -2760,13 +2761,16 @@ __device__ __forceinline__ void mx_chunk16(const uint8_t *W, const uint8_t *R, i
     mx_block16<TYPE, NQ, 7, SC, NT, TS>(st, acc, cr);
 }
 
-/* A word of a staged Q6_K row at byte off past the row's 4-byte-aligned LDS base (O = 2: the
- * super-block sits 2 bytes in, so the word straddles two aligned words). */
+/* A word of a staged Q6_K row at byte off past the row's LDS base. O = 0, 2: the base is 4-byte
+ * aligned and the super-block sits O bytes in (2: the word straddles two aligned words); O = 1:
+ * it sits sh = 0 or 2 bytes in, by the lane's row (rows of an odd number of super-blocks; single
+ * reads at 2-byte alignment cost four times as much). */
 template <int O>
-__device__ __forceinline__ uint32_t q6_word(LdsPtr base, int off)
+__device__ __forceinline__ uint32_t q6_word(LdsPtr base, int off, uint32_t sh)
 {
     typedef __attribute__((address_space(3))) const uint32_t LdsU32;
     if constexpr (O == 0) return *(LdsU32 *)(base + off);
+    else if constexpr (O == 1) return __builtin_amdgcn_alignbyte(*(LdsU32 *)(base + off + 4), *(LdsU32 *)(base + off), sh);
     else return __builtin_amdgcn_alignbyte(*(LdsU32 *)(base + off + 2), *(LdsU32 *)(base + off - 2), 2);
 }
 
@@ -2775,13 +2779,13 @@ __device__ __forceinline__ uint32_t q6_word(LdsPtr base, int off)
  * shift is a constant. The 6-bit code dword is the low nibbles (shifted down for the upper
  * two blocks of a half) with the two high bits of qh moved to bits 4-5 (src/kernels.c:148-160). */
 template <int O, int B, int TS>
-__device__ __forceinline__ MxB mx_weights_q6(LdsPtr q, LdsPtr rb, int t, int kh)
+__device__ __forceinline__ MxB mx_weights_q6(LdsPtr q, LdsPtr rb, int t, int kh, uint32_t sh)
 {
-    constexpr int WS = mx_wstride(14), h = B >> 2, g = B & 3, ns = 4 * (g >> 1), hs = 2 * g;
-    constexpr int oql = O + 64 * h + 32 * (g & 1), oqh = O + 128 + 32 * h;
+    constexpr int WS = mx_wstride(14), h = B >> 2, g = B & 3, ns = 4 * (g >> 1), hs = 2 * g, OO = O == 1 ? 0 : O;
+    constexpr int oql = OO + 64 * h + 32 * (g & 1), oqh = OO + 128 + 32 * h;
     const uint32_t lo4 = 0x0f0f0f0fu;
     auto code = [&](int dq) {
-        const uint32_t ql = q6_word<O>(q, TS * t * WS + oql + dq), qh = q6_word<O>(q, TS * t * WS + oqh + dq);
+        const uint32_t ql = q6_word<O>(q, TS * t * WS + oql + dq, sh), qh = q6_word<O>(q, TS * t * WS + oqh + dq, sh);
         uint32_t hi;
         if constexpr (hs < 4) hi = (qh << (4 - hs)) & 0x30303030u;
         else if constexpr (hs == 4) hi = qh & 0x30303030u;
@@ -2794,7 +2798,7 @@ __device__ __forceinline__ MxB mx_weights_q6(LdsPtr q, LdsPtr rb, int t, int kh)
      * low bytes of its halves (one byte permute each) */
     w.op = __builtin_bit_cast(f16x8, u32x4{ __builtin_amdgcn_perm(cA, cA, 0x0c020c00u), __builtin_amdgcn_perm(cA, cA, 0x0c030c01u),
                                             __builtin_amdgcn_perm(cB, cB, 0x0c020c00u), __builtin_amdgcn_perm(cB, cB, 0x0c030c01u) });
-    const uint32_t scw = *(const __attribute__((address_space(3))) uint16_t *)(rb + TS * t * WS + O + 192 + 8 * h + 2 * g);
+    const uint32_t scw = *(const __attribute__((address_space(3))) uint16_t *)(rb + TS * t * WS + OO + 192 + 8 * h + 2 * g);
     /* the int16 pair {sc[2g], sc[2g+1]}: byte permute with sign fills (selector 10: the sign of
      * byte 1 of the first source, scw << 8, i.e. of sc[2g]; selector 8: of byte 1 of scw) */
     w.sab = __builtin_amdgcn_perm(scw << 8, scw, 0x08010a00u);
@@ -2804,7 +2808,7 @@ __device__ __forceinline__ MxB mx_weights_q6(LdsPtr q, LdsPtr rb, int t, int kh)
     const float s1 = __builtin_fmaf((float)((sx >> 8) & 0xffu), 16777216.0f, -2147483648.0f);
     w.sc = kh ? s1 : s0;
     w.sc1 = s1;
-    w.dw = *(const __attribute__((address_space(3))) uint16_t *)(rb + TS * t * WS + O + 208);
+    w.dw = *(const __attribute__((address_space(3))) uint16_t *)(rb + TS * t * WS + OO + 208);
     return w;
 }
 
@@ -2815,7 +2819,7 @@ __device__ __forceinline__ void mx_block_q6(const MxStreams &st, int kh, f32x4 (
     constexpr int RS = mx_rstride(14), RB = B * mx_recl(14);
     MxB w[2];
 #pragma unroll
-    for (int t = 0; t < 2; t++) w[t] = mx_weights_q6<O, B, TS>(st.q, st.dw, t, kh);
+    for (int t = 0; t < 2; t++) w[t] = mx_weights_q6<O, B, TS>(st.q, st.dw, t, kh, st.sh);
 #pragma unroll
     for (int p = 0; p < NP; p++) {
         /* volatile: keeps each A read a single read into the MFMA operand (records 832 bytes
@@ -2843,7 +2847,7 @@ __device__ __forceinline__ void mx_block_q6(const MxStreams &st, int kh, f32x4 (
 /* A staged Q6_K super-block, its 8 blocks unrolled (offsets and shifts depend on the block);
  * the wave's two tiles TS staged rows apart. */
 template <int NP, int O, int TS>
-__device__ __forceinline__ void mx_chunk_q6(const uint8_t *W, const uint8_t *R, int lr, int lg, int kh, int jd,
+__device__ __forceinline__ void mx_chunk_q6(const uint8_t *W, uint32_t off, const uint8_t *R, int lr, int lg, int kh, int jd,
                                             int offa_lo, int offa_hi, f32x4 (&acc)[2][kMxNA], float (&cr)[2][4])
 {
     constexpr int WS = mx_wstride(14);
@@ -2851,8 +2855,9 @@ __device__ __forceinline__ void mx_chunk_q6(const uint8_t *W, const uint8_t *R, 
     st.alo = (LdsPtr)(R + offa_lo);
     st.ahi = (LdsPtr)(R + offa_hi);
     st.d = (LdsPtr)(R + jd * mx_rstride(14) + kMxDx);
-    st.q = (LdsPtr)(W + lr * WS + 4 * lg);
-    st.dw = (LdsPtr)(W + lr * WS);
+    st.q = (LdsPtr)(W + lr * WS + 4 * lg + (O == 1 ? off & 4u : 0u));
+    st.dw = (LdsPtr)(W + lr * WS + (O == 1 ? off : 0u));
+    st.sh = off & 2u;                          /* O = 1: the super-block's offset in the row */
     mx_opaque(st);
     mx_block_q6<NP, O, 0, TS>(st, kh, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
@@ -2883,7 +2888,7 @@ __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[
     float sc[2][2];
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        w[t] = mx_weights_q6<O, B, TS>(st.q, st.dw, t, 0);
+        w[t] = mx_weights_q6<O, B, TS>(st.q, st.dw, t, 0, st.sh);
         b[t][0] = __builtin_shufflevector(w[t].op, w[t].op, 0, 1, 2, 3);
         b[t][1] = __builtin_shufflevector(w[t].op, w[t].op, 4, 5, 6, 7);
         sc[t][0] = w[t].sc;                                              /* sc[2g] 2^24 */
@@ -2932,7 +2937,7 @@ __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[
 
 /* A staged Q6_K super-block on the 16x16x16 instructions, its 8 blocks unrolled. */
 template <int NQ, int O, int NT, int TS>
-__device__ __forceinline__ void mx_chunk16_q6(const uint8_t *W, const uint8_t *R, int lr, int lg, int offa_lo,
+__device__ __forceinline__ void mx_chunk16_q6(const uint8_t *W, uint32_t off, const uint8_t *R, int lr, int lg, int offa_lo,
                                               int offa_hi, f32x4 (&acc)[2][kMxNA], float (&cr)[2][4])
 {
     constexpr int WS = mx_wstride(14);
@@ -2940,8 +2945,9 @@ __device__ __forceinline__ void mx_chunk16_q6(const uint8_t *W, const uint8_t *R
     st.alo = (LdsPtr)(R + offa_lo);
     st.ahi = (LdsPtr)(R + offa_hi);
     st.d = (LdsPtr)(R + lg * mx_rstride(14) + kMxDx);
-    st.q = (LdsPtr)(W + lr * WS + 4 * lg);
-    st.dw = (LdsPtr)(W + lr * WS);
+    st.q = (LdsPtr)(W + lr * WS + 4 * lg + (O == 1 ? off & 4u : 0u));
+    st.dw = (LdsPtr)(W + lr * WS + (O == 1 ? off : 0u));
+    st.sh = off & 2u;                          /* O = 1: the super-block's offset in the row */
     mx_opaque(st);
     mx_block16_q6<NQ, O, 0, NT, TS>(st, acc, cr);
     __builtin_amdgcn_sched_barrier(0);
@@ -2982,9 +2988,6 @@ __device__ __forceinline__ void mx_wait_barrier()
 #ifndef QMSG_MX_NARROW_GU
 #define QMSG_MX_NARROW_GU 8
 #endif
-#ifndef QMSG_MX_NARROW_DN
-#define QMSG_MX_NARROW_DN 8
-#endif
 #ifndef QMSG_MX_MID_NB
 #define QMSG_MX_MID_NB 2
 #endif
@@ -3015,7 +3018,8 @@ constexpr int mx_waves()
 }
 
 /* Gate/up (MODE 1: gate rows against the token's input records, the same up rows, SwiGLU, the
- * int8 activation blocks and their records) or down (MODE 0: dn rows) of one slot tile, or the rows
+ * int8 activation blocks and their records) or down (MODE 0: dn rows; 3: Q6_K rows of an odd number
+ * of super-blocks, every other one 2 bytes off a word boundary) of one slot tile, or the rows
  * of a dense product (MODE 2: the matrix whose block range holds blockIdx.x, every token a slot,
  * the last block of a matrix moved up to whole rows and storing only those past the one before), with NB
  * staging buffers: 2 (the next chunk's copy in flight while this one computes) or 1 (copy, wait,
@@ -3028,7 +3032,8 @@ void mx_kernel(MxArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem[];
     using Lay = MxLayout<TYPE, WSG, PPW, NW, NT>;
-    constexpr bool GU = MODE == 1, DENSE = MODE == 2;
+    constexpr bool GU = MODE == 1, DENSE = MODE == 2, ODD6 = MODE == 3;
+    static_assert(!ODD6 || (TYPE == 14 && NT == 1), "Q6_K down rows on one-tile waves");
     static_assert(NT == 2 || (NT == 1 && !(GU && TYPE == 14)), "Q6_K gate/up steps two-tile rows");
     /* Q6_K gate/up (4-byte DMA units) steps through its gate rows, then its up rows */
     constexpr bool QS6 = GU && TYPE == 14;
@@ -3125,7 +3130,9 @@ void mx_kernel(MxArgs a)
      * at rbase */
     auto issue_w = [&](int c, uint8_t *base) {
         if constexpr (TYPE == 14) {
-            /* the super-block starts 2 bytes past a 4-byte boundary on odd chunks */
+            /* the super-block starts 2 bytes past a 4-byte boundary on odd chunks (and, down rows
+             * of an odd number of super-blocks, on odd rows: 4 bytes past the copy's start on
+             * odd chunks of odd rows) */
             const uint32_t cb = (uint32_t)(c * 210 - 2 * (c & 1));
             uint32_t o = qoff[0];
             int u = qu;
@@ -3139,7 +3146,7 @@ void mx_kernel(MxArgs a)
                     u = qu_up;
                     wq = wb1;
                 }
-                dma_to_lds<4>(wq + (o + cb), base + 256 * q);
+                dma_to_lds<4>(wq + ((ODD6 ? o & ~3u : o) + cb), base + 256 * q);
                 u += SU;
                 o += SR * rb + 4 * SU;
                 if (u >= Lay::WUR) {
@@ -3247,14 +3254,16 @@ void mx_kernel(MxArgs a)
                 const uint8_t *Wl = (NB == 3 ? smem + buf * Lay::WBYTES : smem + buf * BUF) +
                                     ((GSEP ? 16 : 16 * NT) * wr) * WS;
                 const uint8_t *Rl = (NB == 3 ? rarea : smem + buf * BUF + Lay::WBYTES) + (2 * PPW * ws) * Lay::RS;
+                constexpr int TS6 = QS6 ? RWG / 2 : 16;
                 if constexpr (TYPE == 14 && X16) {
-                    constexpr int TS6 = QS6 ? RWG / 2 : 16;
-                    if (c & 1) mx_chunk16_q6<NP / 2, 2, NT, TS6>(Wl, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
-                    else mx_chunk16_q6<NP / 2, 0, NT, TS6>(Wl, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
+                    if constexpr (ODD6)
+                        mx_chunk16_q6<NP / 2, 1, NT, TS6>(Wl, 2 * (lr & 1) + 2 * (c & 1), Rl, lr, lg, offq_lo, offq_hi, acc, cr);
+                    else if (c & 1) mx_chunk16_q6<NP / 2, 2, NT, TS6>(Wl, 0, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
+                    else mx_chunk16_q6<NP / 2, 0, NT, TS6>(Wl, 0, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
                 } else if constexpr (TYPE == 14) {
-                    constexpr int TS6 = QS6 ? RWG / 2 : 16;
-                    if (c & 1) mx_chunk_q6<NP, 2, TS6>(Wl, Rl, lr, lg, kh, jd, offa_lo, offa_hi, acc, cr);
-                    else mx_chunk_q6<NP, 0, TS6>(Wl, Rl, lr, lg, kh, jd, offa_lo, offa_hi, acc, cr);
+                    static_assert(!ODD6, "rows of alternating alignment run quads");
+                    if (c & 1) mx_chunk_q6<NP, 2, TS6>(Wl, 0, Rl, lr, lg, kh, jd, offa_lo, offa_hi, acc, cr);
+                    else mx_chunk_q6<NP, 0, TS6>(Wl, 0, Rl, lr, lg, kh, jd, offa_lo, offa_hi, acc, cr);
                 } else if constexpr (X16) {
                     mx_chunk16<TYPE, NP / 2, SC, NT, GSEP ? RWG / 2 : 16>(Wl, Rl, lr, lg, offq_lo, offq_hi, acc, cr);
                 } else {
@@ -3391,33 +3400,37 @@ static_assert(2 * mx_lds_bytes(14, 2) <= 160 * 1024, "two Q6_K blocks per CU");
  *          against 350 / 158 at r = 8, 353 / 171 against 422 / 196 at 10, 384 / 186 against
  *          403 / 213 at 12, 719 / 348 against 734 / 364 at 24; 286 / 138 against 275 / 128 at
  *          6 and 262 / 125 against 239 / 114 at 4, where it is not taken;
- *   wide   (other types: gate/up r >= 12, down r >= 16): 8 waves, 4 row groups x 2 slot groups of 4 pairs:
- *          128 rows x 16 slots, two staging buffers;
+ *   wide   (Q6_K gate/up r >= 12): 8 waves, 4 row groups x 2 slot groups of 4 pairs: 128 rows x 16
+ *          slots, two staging buffers;
  *   mid:   4 waves, 4 row groups x 1 slot group of 4 pairs: 128 rows x 8 slots; Q4_0 / Q4_1
  *          two staging buffers (three blocks per CU: the 64-token stack's gate/up 231-233 us
  *          against 235-242 with one), Q6_K one (four blocks per CU);
- *   narrow (Q4_0 / Q4_1 gate/up and down r < 2, Q6_K gate/up r < 3, Q6_K down r < 2.5): 4 waves,
- *          4 row groups x 1 slot group of 2 pairs (128 rows x 4 slots), two buffers (Q6_K down:
- *          one). With the double-buffered mid blocks, Q4_0 narrow / mid (us, gate/up, down):
- *          126-131 / 133, 64-66 / 67 at r = 1; 165 / 165-166, 82 / 82 at 1.5; 188 / 186-187,
- *          92 / 91 at 2; 207-208 / 201-202, 100.5 / 97 at 2.5.
- * Measured per layer at the 235B shape with one-buffer mid blocks (us): gate/up narrow / mid 166 / 178 at r = 1.5, 187 /
- * 199 at 2, 236 / 237 at 3, 287 / 269 at 4; mid / 8-slot blocks of 8 waves 317-325 / 364-378 at
- * 6; mid / wide 407-416 / 460-467 at 8, 571-620 / 581-593 at 12 (run to run), 765-786 / 723-751
- * at 16. Down narrow / mid: Q4_0 89 / 100 at 1.5, 124 / 133 at 3, 154 / 150 at 4; Q6_K 198 /
- * 200 at 1.5, 223 / 223 at 2, 288 / 271 at 3. Down mid / wide: Q4_0 193 / 229 at 8, 271 / 288 at
- * 12, 373 / 375 at 16; Q6_K 362 / 460 at 8, 496 / 549 at 12, 701 / 719 at 16. */
-constexpr int kMxWideSlots = 16;
+ *   narrow (Q4_0 / Q4_1 gate/up r < 2, Q6_K gate/up r < 3): 4 waves, 4 row groups x 1 slot group
+ *          of 2 pairs (128 rows x 4 slots), two buffers. With the double-buffered mid blocks,
+ *          Q4_0 gate/up narrow / mid (us): 126-131 / 133 at r = 1; 165 / 165-166 at 1.5; 188 /
+ *          186-187 at 2; 207-208 / 201-202 at 2.5;
+ *   thin   (down, Q4_0 / Q4_1 r < 8, Q6_K r < 6): 4 waves of one 16-row tile x 4 pairs: 64 rows x 8
+ *          slots, two buffers. Against the narrow and mid blocks down took before (235B, us): Q4_0
+ *          43 / 45 at 8 tokens, 66 / 67 at 16, 84 / 89 at 32, 108 / 108 at 64 (30B 20 / 23 at
+ *          16, 32 / 34 at 64); Q6_K, whose two-tile waves spilled, 78 / 83, 103 / 110, 141 /
+ *          152, 184 / 205. Gate/up gained nothing this way (174 / 171 at 32 tokens);
+ *   Q6_K down r >= 6: 4 waves of one tile x 8 pairs (64 rows x 16 slots, weights in two buffers and
+ *          records in one): 243 / 298 at 128 tokens, 418 / 573 at 256, 759 / 994 at 512 against
+ *          the mid and wide blocks; thin blocks 274, 524, 950 there.
+ * Measured per layer at the 235B shape with one-buffer mid blocks (us): gate/up narrow / mid 166 /
+ * 178 at r = 1.5, 187 / 199 at 2, 236 / 237 at 3, 287 / 269 at 4; mid / 8-slot blocks of 8 waves
+ * 317-325 / 364-378 at 6; mid / wide 407-416 / 460-467 at 8, 571-620 / 581-593 at 12 (run to run),
+ * 765-786 / 723-751 at 16. */
 constexpr int kMxWideSlotsGateUp = 12;
-enum MxShape { kMxNarrow, kMxMid, kMxWide, kMxWide16 };
+enum MxShape { kMxNarrow, kMxMid, kMxWide, kMxWide16, kMxThin };
 
 static MxShape mx_shape(const Shape &s, int T, int gu, int type)
 {
     const long NS = (long)T * s.K, act = s.X < NS ? s.X : NS;
-    const long wide_slots = gu ? kMxWideSlotsGateUp : kMxWideSlots;
+    if (!gu && NS < (type == 14 ? 6 : QMSG_MX_WIDE16_SLOTS) * act) return kMxThin;
     if (type != 14 && QMSG_MX_WIDE16_SLOTS > 0 && NS >= QMSG_MX_WIDE16_SLOTS * act) return kMxWide16;
-    if (NS >= wide_slots * act) return kMxWide;
-    const long narrow_quarters = type == 14 ? (gu ? 12 : 10) : (gu ? QMSG_MX_NARROW_GU : QMSG_MX_NARROW_DN);
+    if (NS >= kMxWideSlotsGateUp * act) return kMxWide;
+    const long narrow_quarters = type == 14 ? 12 : QMSG_MX_NARROW_GU;
     return 4 * NS < narrow_quarters * act ? kMxNarrow : kMxMid;
 }
 
@@ -3437,8 +3450,8 @@ static void launch_mx_shape(const MxArgs &a, int rows, int maxt, hipStream_t st)
                 dim3(64 * NW), lds, st, b);
         return;
     }
-    QLAUNCH(GU ? "gateup" : "down", (mx_kernel<TYPE, WSG, GU, PPW, NW, NB, NT>),
-            dim3(rows / (GU ? Lay::RWG / 2 : Lay::RWG), maxt, kTileN / Lay::SWG), dim3(64 * NW), lds, st, a);
+    QLAUNCH(GU == 1 ? "gateup" : "down", (mx_kernel<TYPE, WSG, GU, PPW, NW, NB, NT>),
+            dim3(rows / (GU == 1 ? Lay::RWG / 2 : Lay::RWG), maxt, kTileN / Lay::SWG), dim3(64 * NW), lds, st, a);
 }
 
 /* Other shapes of the same kernel measured at the 512-token prefill: 32-slot blocks of 16
@@ -3453,6 +3466,14 @@ static void launch_mx_shape(const MxArgs &a, int rows, int maxt, hipStream_t st)
 template <int TYPE, int GU>
 static void launch_mx(const MxArgs &a, int rows, int maxt, MxShape shape, hipStream_t st)
 {
+    if constexpr (!GU) {
+        if constexpr (TYPE == 14) {
+            if (a.rb % 4 && shape == kMxThin) return launch_mx_shape<14, 3, 1, 4, 4, 2, 1>(a, rows, maxt, st);
+            if (a.rb % 4) return launch_mx_shape<14, 3, 1, 8, 4, 3, 1>(a, rows, maxt, st);
+        }
+        if (shape == kMxThin) return launch_mx_shape<TYPE, 0, 1, 4, 4, 2, 1>(a, rows, maxt, st);
+        if constexpr (TYPE == 14) return launch_mx_shape<14, 0, 1, 8, 4, 3, 1>(a, rows, maxt, st);
+    }
     if (shape == kMxWide) launch_mx_shape<TYPE, GU, 2, 4, 8>(a, rows, maxt, st);
     else if (shape == kMxWide16) {
         /* Q4_0 / Q4_1 only (mx_shape) */
@@ -3462,20 +3483,19 @@ static void launch_mx(const MxArgs &a, int rows, int maxt, MxShape shape, hipStr
         else if constexpr (TYPE != 14)
             launch_mx_shape<TYPE, GU, 1, 8, 4, GU ? QMSG_MX_WIDE16_NB_GU : QMSG_MX_WIDE16_NB_DN>(a, rows, maxt, st);
     }
-    else if (shape == kMxNarrow) launch_mx_shape<TYPE, GU, 1, 2, 4, (!GU && TYPE == 14) ? 1 : 2>(a, rows, maxt, st);
+    else if (shape == kMxNarrow) launch_mx_shape<TYPE, GU, 1, 2, 4, 2>(a, rows, maxt, st);
     else launch_mx_shape<TYPE, GU, 1, 4, 4, TYPE == 14 ? QMSG_MX_MID_NB_Q6 : QMSG_MX_MID_NB>(a, rows, maxt, st);
 }
 
 /* Whether the MFMA kernels take this layer: gate and up of one type (Q4_0, Q4_1, or Q6_K with
- * rows a multiple of 4 bytes long); Q4_0, Q4_1 or Q6_K down (Q6_K
- * rows a multiple of 4 bytes long); 32-blocks in whole chunks; rows in whole blocks' tiles. */
+ * rows a multiple of 4 bytes long); Q4_0, Q4_1 or Q6_K down; 32-blocks in whole chunks; rows in whole blocks' tiles. */
 bool mx_supported(const Shape &s, const LayerDev &L, int *down_mx)
 {
     const int nbE = s.E / 32, nbF = s.F / 32;
     const bool gu = L.gate_type == L.up_type &&
                     (L.gate_type == 2 || L.gate_type == 3 || (L.gate_type == 14 && L.gate_rb % 4 == 0)) &&
                     nbE % kMxC == 0 && s.F % 128 == 0 && (uint64_t)s.F * L.gate_rb < (1ull << 31);
-    const bool dn = (L.down_type == 2 || L.down_type == 3 || (L.down_type == 14 && L.down_rb % 4 == 0)) &&
+    const bool dn = (L.down_type == 2 || L.down_type == 3 || L.down_type == 14) &&
                     nbF % kMxC == 0 && s.E % 256 == 0 && (uint64_t)s.E * L.down_rb < (1ull << 31);
     if (down_mx) *down_mx = dn;
     return gu;
@@ -3613,7 +3633,7 @@ static void launch_dense_mx_type(const MxArgs &a, hipStream_t st)
         if (a.d.T <= 32) launch_mx_shape<14, 2, 1, 2, 4, 2, 1>(a, 0, 0, st);
         else if (a.d.T < 96) launch_mx_shape<14, 2, 1, 4, 4, 2, 1>(a, 0, 0, st);
         else if (blocks < 2048) launch_mx_shape<14, 2, 2, 4, 8, 2, 1>(a, 0, 0, st);
-        else launch_mx_shape<14, 2, 1, 8, 4, 1, 1>(a, 0, 0, st);
+        else launch_mx_shape<14, 2, 1, 8, 4, 3, 1>(a, 0, 0, st);
     } else {
         if (a.d.T <= 64) launch_mx_shape<TYPE, 2, 1, 2, 4, 2, 1>(a, 0, 0, st);
         else if (blocks < 1536) launch_mx_shape<TYPE, 2, 2, 4, 8, 2, 1>(a, 0, 0, st);
