@@ -24,7 +24,7 @@
  * Bound: the matrix pipe at batch sizes (padding of partly filled 16-column tiles included), the
  * one chain's latency at one token. The 30B shape with Q8_0 experts, us, against one lane per row
  * and four slots per pass on the vector ALU: gate/up with SwiGLU 19 (45 + 7), down 9.8 (20) at
- * one token; 257 and 137 (together 5744) at 201 tokens of a skewed load, the layer 393 (5860). */
+ * one token; 254 and 135 (together 5744) at 201 tokens of a skewed load, the layer 383 (5860). */
 #include <type_traits>
 
 #include "qmsg_device.h"
@@ -59,10 +59,8 @@ struct ChRaw {
     uint32_t s, s2;
 };
 
-/* Reads at the rows' alignment (2 bytes for Q8_0, Q4_0 and Q6_K blocks). */
+/* Global reads at the rows' alignment (2 bytes for Q8_0, Q4_0 and Q6_K blocks). */
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
-typedef uint32_t u32_a2 __attribute__((aligned(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 /* Lane group g's quarter of block b (a constant) of the staged row at p. */
@@ -83,14 +81,21 @@ __device__ __forceinline__ void ch_read(const uint8_t *p, int b, int g, ChRaw<TY
         r.q[2] = v1.x;
         r.q[3] = v1.y;
     } else if constexpr (TYPE == 8) {
-        const u32x2 v = *(const u32x2_a2 *)(p + 34 * b + 8 * g + 2);
-        r.q[0] = v.x;
-        r.q[1] = v.y;
+        /* even blocks' codes sit 2 bytes past a word: aligned words and a byte shift (LDS reads
+         * off their alignment are several times slower) */
+        const uint32_t *w = (const uint32_t *)(p + 34 * b + 8 * g + ((b & 1) ? 2 : 0));
+        if (b & 1) {
+            r.q[0] = w[0];
+            r.q[1] = w[1];
+        } else {
+            r.q[0] = __builtin_amdgcn_alignbyte(w[1], w[0], 2);
+            r.q[1] = __builtin_amdgcn_alignbyte(w[2], w[1], 2);
+        }
         r.s = *(const uint16_t *)(p + 34 * b);
     } else if constexpr (TYPE == 14) {
         const int hf = (b & 7) >> 2, gb = b & 3;
-        const u32x2 lo = *(const u32x2_a2 *)(p + 64 * hf + 32 * (gb & 1) + 8 * g);
-        const u32x2 hi = *(const u32x2_a2 *)(p + 128 + 32 * hf + 8 * g);
+        const u32x2 lo = *(const u32x2 *)(p + 64 * hf + 32 * (gb & 1) + 8 * g);
+        const u32x2 hi = *(const u32x2 *)(p + 128 + 32 * hf + 8 * g);
         r.q[0] = lo.x;
         r.q[1] = lo.y;
         r.q[2] = hi.x;
@@ -102,7 +107,8 @@ __device__ __forceinline__ void ch_read(const uint8_t *p, int b, int g, ChRaw<TY
         r.q[0] = *(const uint32_t *)(p + 20 * b + 4 * g + 4);
     } else {
         r.s = *(const uint16_t *)(p + 18 * b);
-        r.q[0] = *(const u32_a2 *)(p + 18 * b + 4 * g + 2);
+        const uint32_t *w = (const uint32_t *)(p + 18 * b + 4 * g + ((b & 1) ? 2 : 0));
+        r.q[0] = (b & 1) ? w[0] : __builtin_amdgcn_alignbyte(w[1], w[0], 2);
     }
 }
 
