@@ -87,6 +87,10 @@ std::vector<ScratchItem> scratch_items(const qmsg_cfg &cfg, size_t T, Scratch *S
  * process ends. Host code never passes `scratch` itself (in host code the name is only a
  * stand-in): each device's address comes from hipGetSymbolAddress, taken once per device
  * with that device current (in qmsg_create), and only that address is used. */
+/* Host-buffer layer calls of up to this many input bytes pass through pinned memory that the kernels
+ * read and write themselves (qmsg_moe). */
+constexpr size_t kHostStage = 256 * 1024;
+
 constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;
 constexpr int kMaxDevices = 64;
 __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
@@ -143,6 +147,8 @@ struct qmsg_ctx {
     size_t dense_xqk_bytes = 0;
     void *dense_io = nullptr;
     size_t dense_io_bytes = 0;
+    /* pinned rows of the host-buffer layer call (kHostStage bytes in, as many out), on first use */
+    uint8_t *pin = nullptr;
     std::string err;
     bool prof = false;
     std::vector<ProfRec> prof_recs, prof_free;
@@ -281,6 +287,7 @@ void qmsg_destroy(qmsg_ctx *c)
     for (auto &m : c->mats) hipFree(m.w);
     hipFree(c->dense_xqk);
     hipFree(c->dense_io);
+    if (c->pin) hipHostFree(c->pin);
     for (void *p : c->scratch_allocs) hipFree(p);
     for (void *p : c->user_allocs) hipFree(p);
     for (auto &r : c->prof_recs) { hipEventDestroy(r.a); hipEventDestroy(r.b); }
@@ -1038,6 +1045,24 @@ int qmsg_moe(qmsg_ctx *c, int layer, const float *xn, const float *h, int T, flo
     if (!xn || !out) return fail(c, QMSG_E_INVALID, "qmsg_moe: null buffer");
     const size_t bytes = (size_t)T * c->cfg.n_embd * 4;
     HIP_TRY(c, hipSetDevice(c->device));
+    /* Small calls: the input through pinned memory and a copy kernel, and the layer's last launch
+     * stores its rows to pinned memory. Pageable copies cost a runtime blit and a host round
+     * trip each. us per call, pinned / pageable: 30B 40 / 56 at one token, 85 / 126 at 8, 147 / 186
+     * at 32 (256 KiB in); 235B 50 / 59, 171 / 213, 255 / 298 at 16 (256 KiB). */
+    if (bytes <= kHostStage && !c->pin && hipHostMalloc((void **)&c->pin, 2 * kHostStage, hipHostMallocDefault) != hipSuccess) {
+        c->pin = nullptr;                     /* the pageable copies below */
+        (void)hipGetLastError();
+    }
+    if (bytes <= kHostStage && c->pin) {
+        memcpy(c->pin, xn, bytes);
+        LAUNCH(c, "copy", launch_copy(c->d_x, c->pin, bytes, c->stream));
+        const int rc = run_layer(c, layer, c->d_x, T, (float *)(c->pin + kHostStage), 0);
+        /* also after an error: the copy still reads the pinned rows */
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        if (rc) return rc;
+        memcpy(out, c->pin + kHostStage, bytes);
+        return QMSG_OK;
+    }
     HIP_TRY(c, hipMemcpyAsync(c->d_x, xn, bytes, hipMemcpyHostToDevice, c->stream));
     int rc = run_layer(c, layer, c->d_x, T, c->d_out, 0);
     if (rc) return rc;
