@@ -780,6 +780,8 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
         return fail(c, QMSG_E_UNSUPPORTED, "qmsg_matmul_n: fp32-chain rows above %d columns", 160 * 1024 / 4);
     /* launches of up to kDenseMats matrices of one type, in argument order */
     std::vector<bool> done((size_t)nW, false);
+    const uint64_t epoch = next_epoch();
+    bool records = false;
     for (int i = 0; i < nW; i++) {
         if (done[(size_t)i]) continue;
         const int type = c->mats[(size_t)ids[i]].type;
@@ -798,7 +800,7 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
             done[(size_t)j] = true;
         }
         if (exact) LAUNCH(c, "dense", launch_dense_exact(a, type, c->stream));
-        else LAUNCH(c, "dense", launch_dense(a, type, (uint8_t *)c->dense_xqk, next_epoch(), c->stream));
+        else LAUNCH(c, "dense", launch_dense(a, type, (uint8_t *)c->dense_xqk, epoch, &records, c->stream));
     }
     return QMSG_OK;
 }

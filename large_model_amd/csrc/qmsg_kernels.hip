@@ -2069,11 +2069,11 @@ __global__ __launch_bounds__(32 * RD) void down_small_kernel(DownArgs a)
 
 /* The int8 blocks of every slot's activations (src/model.c:996-997) for batches whose
  * records do not fit the down kernel's LDS: one thread per 32-block. */
-__device__ bool mx_store_record(const Q8Vals &q, uint8_t *rec, bool hi16);
+__device__ bool mx_store_record(const Q8Vals &q, uint8_t *rec);
 
 /* The int8 activation blocks of every slot (src/model.c:996-997) from act: QmsQ8 blocks, pair
  * records, and, when mxrec is set, the MFMA kernels' records too. */
-__global__ void act_quant_kernel(Scratch S, int F, int NS, uint8_t *mxrec, int hi16)
+__global__ void act_quant_kernel(Scratch S, int F, int NS, uint8_t *mxrec)
 {
     const int nbF = F >> 5;
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2089,7 +2089,7 @@ __global__ void act_quant_kernel(Scratch S, int F, int NS, uint8_t *mxrec, int h
     const Q8Vals q = quantize_block(v);
     store_q8(q, S.aq + b);
     store_pair_half(q, (uint32_t *)(S.aqk + ((size_t)s * (nbF >> 1) + (blk >> 1)) * kPairBytes), blk & 1);
-    if (mxrec && !mx_store_record(q, mxrec + (size_t)b * kMxRec, hi16)) S.mxflag[1] = S.epoch;
+    if (mxrec && !mx_store_record(q, mxrec + (size_t)b * kMxRec)) S.mxflag[1] = S.epoch;
 }
 
 /* Weighted sum per token in selection order (src/model.c:1152-1162) when dn did not fit. */
@@ -2232,7 +2232,7 @@ hipError_t launch_down_exact(const Shape &s, const LayerDev &L, const Scratch &S
     const bool qa = quant && T <= kTileQuantT;
     if (quant && !qa) {
         const int nq = NS * (s.F / 32);
-        QLAUNCH("actq", act_quant_kernel, dim3((nq + 255) / 256), dim3(256), 0, st, S, s.F, NS, (uint8_t *)nullptr, 0);
+        QLAUNCH("actq", act_quant_kernel, dim3((nq + 255) / 256), dim3(256), 0, st, S, s.F, NS, (uint8_t *)nullptr);
     }
     const int NT = T >= 4 ? 4 : (T >= 2 ? 2 : 1);
     const int RT = L.down_type == 14 ? kDownTileRowsQ6K : 64;
@@ -2378,9 +2378,10 @@ __device__ __forceinline__ float mx_scaled_d(float d)
 }
 
 /* One int8 block as an activation record (layout above); false when its d_x 2^24 word is the
- * NaN (d_x outside the scaled range). hi16: for Q4_0 / Q4_1 rows, whose B operand takes the
- * high nibbles in place (code 16 2^-24), lanes 4-7 carry x / 16 (exact in f16). */
-__device__ bool mx_store_record(const Q8Vals &q, uint8_t *rec, bool hi16)
+ * NaN (d_x outside the scaled range). Lanes 4-7 carry x / 16 (exact in f16): the Q4_0 / Q4_1 B
+ * operand takes the high nibbles in place (code 16 2^-24), and Q6_K folds the 16 into those
+ * lanes' sub-scale, so one set of records serves every row type. */
+__device__ bool mx_store_record(const Q8Vals &q, uint8_t *rec)
 {
     u32x4 w[6];
 #pragma unroll
@@ -2388,7 +2389,7 @@ __device__ bool mx_store_record(const Q8Vals &q, uint8_t *rec, bool hi16)
         const uint32_t c = q.qw[k];
         const int x0 = (int)(int8_t)(c & 0xffu), x1 = (int)(int8_t)((c >> 8) & 0xffu);
         const int x2 = (int)(int8_t)((c >> 16) & 0xffu), x3 = (int)(int8_t)(c >> 24);
-        const float sc = (hi16 && k >= 4) ? 0.0625f : 1.0f;
+        const float sc = k >= 4 ? 0.0625f : 1.0f;
         auto h = [sc](int x) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)((float)x * sc)); };
         w[k >> 1][2 * (k & 1)] = h(x0) | (h(x2) << 16);
         w[k >> 1][2 * (k & 1) + 1] = h(x1) | (h(x3) << 16);
@@ -2402,7 +2403,7 @@ __device__ bool mx_store_record(const Q8Vals &q, uint8_t *rec, bool hi16)
 }
 
 /* The layer input's records from its int8 blocks (one thread per block). */
-__global__ void mx_input_kernel(const Q8 *xq, int n, uint8_t *rec, uint64_t *flag, uint64_t epoch, int hi16)
+__global__ void mx_input_kernel(const Q8 *xq, int n, uint8_t *rec, uint64_t *flag, uint64_t epoch)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -2413,7 +2414,7 @@ __global__ void mx_input_kernel(const Q8 *xq, int n, uint8_t *rec, uint64_t *fla
     q.s16 = s[2];
 #pragma unroll
     for (int w = 0; w < 8; w++) q.qw[w] = s[3 + w];
-    if (!mx_store_record(q, rec + (size_t)i * kMxRec, hi16)) *flag = epoch;
+    if (!mx_store_record(q, rec + (size_t)i * kMxRec)) *flag = epoch;
 }
 
 struct MxArgs {
@@ -2422,7 +2423,6 @@ struct MxArgs {
     int E, F, debug;
     const uint8_t *rec;          /* input records: [token][E/32] (gate/up) or [slot][F/32] (down) */
     uint8_t *rec_out;            /* gate/up: the activation records [slot][F/32] */
-    int rec_out_hi16;            /* gate/up: the down rows are Q4_0 / Q4_1 (records' lanes 4-7 x / 16) */
     Scratch S;
     DenseArgs d;                 /* dense rows: the matrices, T and C (rec: [token][C/32])      */
 };
@@ -2475,9 +2475,9 @@ __device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t m, uint32_t c)
 struct MxB {
     f16x8 op;
     uint32_t dw;      /* Q4_0: d (low half); Q4_1: d | m << 16; Q6_K: d (low half) */
-    float sc;         /* Q6_K: the lane's sub-scale times 2^24 (k < 4: sc[2g], k >= 4: sc[2g+1]) */
+    float sc;         /* Q6_K: the lane's sub-scale times 2^24 (k < 4: sc[2g]) or 2^28 (sc[2g+1]) */
     uint32_t sab;     /* Q6_K: both sub-scales as int16 pair (sc[2g] low) */
-    float sc1;        /* Q6_K: sc[2g+1] times 2^24 */
+    float sc1;        /* Q6_K: sc[2g+1] times 2^28 */
 };
 
 /* a.lo*b.lo + a.hi*b.hi over int16 halves (v_dot2_i32_i16 with a zero addend: no register to
@@ -2805,7 +2805,8 @@ __device__ __forceinline__ MxB mx_weights_q6(LdsPtr q, LdsPtr rb, int t, int kh,
     /* sc * 2^24 = (u - 128) * 2^24 for the byte u = sc ^ 0x80, exact in one fma */
     const uint32_t sx = scw ^ 0x8080u;
     const float s0 = __builtin_fmaf((float)(sx & 0xffu), 16777216.0f, -2147483648.0f);
-    const float s1 = __builtin_fmaf((float)((sx >> 8) & 0xffu), 16777216.0f, -2147483648.0f);
+    /* lanes 4-7: the records carry x / 16 */
+    const float s1 = __builtin_fmaf((float)((sx >> 8) & 0xffu), 268435456.0f, -34359738368.0f);
     w.sc = kh ? s1 : s0;
     w.sc1 = s1;
     w.dw = *(const __attribute__((address_space(3))) uint16_t *)(rb + TS * t * WS + OO + 208);
@@ -2892,7 +2893,7 @@ __device__ __forceinline__ void mx_block16_q6(const MxStreams &st, f32x4 (&acc)[
         b[t][0] = __builtin_shufflevector(w[t].op, w[t].op, 0, 1, 2, 3);
         b[t][1] = __builtin_shufflevector(w[t].op, w[t].op, 4, 5, 6, 7);
         sc[t][0] = w[t].sc;                                              /* sc[2g] 2^24 */
-        sc[t][1] = w[t].sc1;                                             /* sc[2g+1] 2^24 */
+        sc[t][1] = w[t].sc1;                                             /* sc[2g+1] 2^28 */
     }
     f32x4 S[2][2];
     float xd[NQ], dd[2];
@@ -3377,7 +3378,7 @@ void mx_kernel(MxArgs a)
         const int s = s0 + sl, blk = (R0 >> 5) + g;
         store_q8(q, a.S.aq + (size_t)s * nbF + blk);
         store_pair_half(q, (uint32_t *)(a.S.aqk + ((size_t)s * (nbF >> 1) + (blk >> 1)) * kPairBytes), blk & 1);
-        if (!mx_store_record(q, a.rec_out + ((size_t)s * nbF + blk) * kMxRec, a.rec_out_hi16))
+        if (!mx_store_record(q, a.rec_out + ((size_t)s * nbF + blk) * kMxRec))
             a.S.mxflag[1] = a.S.epoch;
     }
 }
@@ -3508,8 +3509,7 @@ hipError_t launch_experts_mx(const Shape &s, const LayerDev &L, const Scratch &S
     if (!mx_supported(s, L, &down_mx)) return hipErrorInvalidValue;
     const int NS = T * s.K, maxt = (s.X < NS ? s.X : NS) + NS / kTileN + 1;
     const int nx = T * (s.E / 32);
-    QLAUNCH("mxin", mx_input_kernel, dim3((nx + 255) / 256), dim3(256), 0, st, S.xq, nx, S.mxx, S.mxflag, S.epoch,
-            L.gate_type != 14 ? 1 : 0);
+    QLAUNCH("mxin", mx_input_kernel, dim3((nx + 255) / 256), dim3(256), 0, st, S.xq, nx, S.mxx, S.mxflag, S.epoch);
     MxArgs a;
     a.w0 = L.gate;
     a.w1 = L.up;
@@ -3520,7 +3520,6 @@ hipError_t launch_experts_mx(const Shape &s, const LayerDev &L, const Scratch &S
     a.debug = debug;
     a.rec = S.mxx;
     a.rec_out = S.mxa;
-    a.rec_out_hi16 = L.down_type != 14 ? 1 : 0;
     a.S = S;
     if (L.gate_type == 14) launch_mx<14, 1>(a, s.F, maxt, mx_shape(s, T, 1, 14), st);
     else if (L.gate_type == 3) launch_mx<3, 1>(a, s.F, maxt, mx_shape(s, T, 1, 3), st);
@@ -3536,7 +3535,6 @@ hipError_t launch_experts_mx(const Shape &s, const LayerDev &L, const Scratch &S
     a.eb = L.down_eb;
     a.rec = S.mxa;
     a.rec_out = nullptr;
-    a.rec_out_hi16 = 0;
     if (L.down_type == 14) launch_mx<14, 0>(a, s.E, maxt, mx_shape(s, T, 0, 14), st);
     else if (L.down_type == 3) launch_mx<3, 0>(a, s.E, maxt, mx_shape(s, T, 0, 3), st);
     else launch_mx<2, 0>(a, s.E, maxt, mx_shape(s, T, 0, 2), st);
@@ -3554,8 +3552,7 @@ hipError_t launch_down_mx(const Shape &s, const LayerDev &L, const Scratch &S, f
     if (!down_mx) return hipErrorInvalidValue;
     const int NS = T * s.K, maxt = (s.X < NS ? s.X : NS) + NS / kTileN + 1;
     const int nq = NS * (s.F / 32);
-    QLAUNCH("actq", act_quant_kernel, dim3((nq + 255) / 256), dim3(256), 0, st, S, s.F, NS, S.mxa,
-            L.down_type != 14 ? 1 : 0);
+    QLAUNCH("actq", act_quant_kernel, dim3((nq + 255) / 256), dim3(256), 0, st, S, s.F, NS, S.mxa);
     MxArgs a;
     a.w0 = L.down;
     a.w1 = nullptr;
@@ -3566,7 +3563,6 @@ hipError_t launch_down_mx(const Shape &s, const LayerDev &L, const Scratch &S, f
     a.debug = 0;
     a.rec = S.mxa;
     a.rec_out = nullptr;
-    a.rec_out_hi16 = 0;
     a.S = S;
     if (L.down_type == 14) launch_mx<14, 0>(a, s.E, maxt, mx_shape(s, T, 0, 14), st);
     else if (L.down_type == 3) launch_mx<3, 0>(a, s.E, maxt, mx_shape(s, T, 0, 3), st);
@@ -3598,7 +3594,7 @@ __global__ void dense_quant_kernel(const float *x, int C, int T, uint8_t *xqk)
 }
 
 /* The same rows' MFMA records (T * C / 32 of kMxRec bytes). */
-__global__ void dense_mx_quant_kernel(const float *x, int n, uint8_t *rec, uint64_t *flag, uint64_t epoch, int hi16)
+__global__ void dense_mx_quant_kernel(const float *x, int n, uint8_t *rec, uint64_t *flag, uint64_t epoch)
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= n) return;
@@ -3609,7 +3605,7 @@ __global__ void dense_mx_quant_kernel(const float *x, int n, uint8_t *rec, uint6
         const float4 f = src[j];
         v[4 * j] = f.x; v[4 * j + 1] = f.y; v[4 * j + 2] = f.z; v[4 * j + 3] = f.w;
     }
-    if (!mx_store_record(quantize_block(v), rec + (size_t)b * kMxRec, hi16)) *flag = epoch;
+    if (!mx_store_record(quantize_block(v), rec + (size_t)b * kMxRec)) *flag = epoch;
 }
 
 /* Dense rows on the MFMA kernels (mx_kernel MODE 2). Most dense grids are small (72 blocks of 128
@@ -3657,7 +3653,8 @@ static bool dense_mx_takes(const DenseArgs &a, int type)
     return a.T > 8 || (a.T > 4 && rows * a.C >= 1l << 24);
 }
 
-static hipError_t launch_dense_mx(const DenseArgs &d, int type, uint8_t *buf, uint64_t epoch, hipStream_t st)
+static hipError_t launch_dense_mx(const DenseArgs &d, int type, uint8_t *buf, uint64_t epoch, bool records,
+                                  hipStream_t st)
 {
     const int n = d.T * (d.C / 32);
     MxArgs a{};
@@ -3666,8 +3663,9 @@ static hipError_t launch_dense_mx(const DenseArgs &d, int type, uint8_t *buf, ui
     a.rec = buf + 256;
     a.S.mxflag = (uint64_t *)buf;
     a.S.epoch = epoch;
-    QLAUNCH("dquant", dense_mx_quant_kernel, dim3((n + 255) / 256), dim3(256), 0, st, d.x, n, buf + 256,
-            a.S.mxflag + 1, epoch, type != 14 ? 1 : 0);
+    if (!records)
+        QLAUNCH("dquant", dense_mx_quant_kernel, dim3((n + 255) / 256), dim3(256), 0, st, d.x, n, buf + 256,
+                a.S.mxflag + 1, epoch);
     if (type == 14) launch_dense_mx_type<14>(a, st);
     else if (type == 3) launch_dense_mx_type<3>(a, st);
     else launch_dense_mx_type<2>(a, st);
@@ -4444,11 +4442,15 @@ hipError_t launch_f32_rows(const float *w, int rows, int C, const float *x, int 
     return hipGetLastError();
 }
 
-hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t epoch, hipStream_t st)
+hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t epoch, bool *records, hipStream_t st)
 {
     DenseArgs a = args;
     const int nb = a.C / 32;
-    if (xqk && dense_mx_takes(a, type)) return launch_dense_mx(a, type, xqk, epoch, st);
+    if (xqk && dense_mx_takes(a, type)) {
+        const bool have = *records;
+        *records = true;
+        return launch_dense_mx(a, type, xqk, epoch, have, st);
+    }
     if (type != 0 && (type == 14 ? nb % 64 != 0 : nb % 8 != 0)) {
         /* widths the chunked kernels do not take: one direct-read pass per NT tokens */
         const int NT = dense_any_nt(type, a.T, nb);
@@ -4486,6 +4488,7 @@ hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t 
     if (a.T >= kDenseQuantT && xqk) {
         QLAUNCH("dquant", dense_quant_kernel, dim3((a.T * nb + 255) / 256), dim3(256), 0, st, a.x, a.C, a.T, xqk);
         a.xqk = xqk;
+        *records = false;                     /* the pair records took their place */
     }
     /* one wave per block, 16 rows each: the trunk's small matrices (attn_k/v: 512 rows) still
      * spread over 32 CUs, the large ones over every CU */
