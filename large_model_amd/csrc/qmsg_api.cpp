@@ -765,8 +765,19 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
     if (T == 0) return QMSG_OK;
     if (!d_x || ((uintptr_t)d_x & 15)) return fail(c, QMSG_E_INVALID, "qmsg_matmul_n: x must be 16-byte aligned");
     HIP_TRY(c, hipSetDevice(c->device));
-    if (T >= kDenseRecordT) {
-        const int rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, dense_record_bytes((size_t)T, (size_t)C));
+    /* The record buffer. Calls of fewer than kDenseQuantT rows can do without it (a captured call,
+     * or no memory: the row kernels), larger ones with the smaller pair records. */
+    bool mfma = T >= kDenseRecordT;
+    if (mfma && c->dense_xqk_bytes < dense_record_bytes((size_t)T, (size_t)C)) {
+        const size_t pairs = (size_t)T * (size_t)(C / 64) * kPairBytes;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (T < kDenseQuantT) HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
+        int rc = cap == hipStreamCaptureStatusNone
+                     ? grow(c, &c->dense_xqk, &c->dense_xqk_bytes, dense_record_bytes((size_t)T, (size_t)C))
+                     : QMSG_E_NOMEM;
+        mfma = rc == QMSG_OK;
+        if (rc == QMSG_E_NOMEM && T < kDenseQuantT) rc = QMSG_OK;
+        else if (rc == QMSG_E_NOMEM) rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, pairs);
         if (rc) return rc;
     }
     /* qms_matmul_n's choice for the whole call (src/quant.c:131-141): the fast loop, or
@@ -800,7 +811,7 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
             done[(size_t)j] = true;
         }
         if (exact) LAUNCH(c, "dense", launch_dense_exact(a, type, c->stream));
-        else LAUNCH(c, "dense", launch_dense(a, type, (uint8_t *)c->dense_xqk, epoch, &records, c->stream));
+        else LAUNCH(c, "dense", launch_dense(a, type, (uint8_t *)c->dense_xqk, epoch, mfma ? &records : nullptr, c->stream));
     }
     return QMSG_OK;
 }

@@ -231,7 +231,7 @@ hipError_t launch_call_reset(const Scratch &S, hipStream_t st);
 /* The dense rows kernel; for T >= kDenseQuantT (MFMA kernels: kDenseRecordT) the input records are formed first into xqk
  * (dense_record_bytes), whose flag word takes epoch (unique per call) when one is outside the
  * MFMA kernels' scaled range. *records: xqk holds the MFMA records of this call's rows (formed by an
- * earlier launch of the call); updated. */
+ * earlier launch of the call); updated. NULL: no MFMA kernels (xqk smaller or NULL). */
 inline size_t dense_record_bytes(size_t T, size_t C) { return 256 + T * (C / 32) * kMxRec; }
 hipError_t launch_dense(const DenseArgs &a, int type, uint8_t *xqk, uint64_t epoch, bool *records, hipStream_t st);
 /* matmul_exact for every matrix of a call (--exact, or an F16 / Q8_0 matrix in the call). */

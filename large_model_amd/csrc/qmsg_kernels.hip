@@ -4446,7 +4446,7 @@ hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t 
 {
     DenseArgs a = args;
     const int nb = a.C / 32;
-    if (xqk && dense_mx_takes(a, type)) {
+    if (records && dense_mx_takes(a, type)) {
         const bool have = *records;
         *records = true;
         return launch_dense_mx(a, type, xqk, epoch, have, st);
@@ -4488,7 +4488,7 @@ hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t 
     if (a.T >= kDenseQuantT && xqk) {
         QLAUNCH("dquant", dense_quant_kernel, dim3((a.T * nb + 255) / 256), dim3(256), 0, st, a.x, a.C, a.T, xqk);
         a.xqk = xqk;
-        *records = false;                     /* the pair records took their place */
+        if (records) *records = false;        /* the pair records took their place */
     }
     /* one wave per block, 16 rows each: the trunk's small matrices (attn_k/v: 512 rows) still
      * spread over 32 CUs, the large ones over every CU */
