@@ -2326,7 +2326,8 @@ hipError_t launch_gateup_tiles(const Shape &s, const LayerDev &L, const Scratch 
  *     so a mask unpacks them (the matrix cores keep subnormal inputs; checked on the device);
  *   - A is block-diagonal over the lane groups: its row (slot j, lane k) holds x_j only at the
  *     four K positions of group k, so D-row (j, k) of column r sums group k only.
- * Every product and partial sum is an integer multiple of 2^-24 below 1, so the f32
+ * Every product and partial sum is an integer multiple of 2^-24 (Q6_K lanes 4-7, against x / 16:
+ * 2^-28) below 1 with at most 16 significant bits, so the f32
  * accumulation inside the MFMA is exact in any order and D equals S_k 2^-24. The VALU then runs
  * the reference's chains, acc_k = fma(S_k, fl(d_w d_x), acc_k) per block, as
  * fma(D, fl(d_w d_x 2^24), acc_k): the record carries d_x 2^24, and for d_x in [2^-102, 2^88]
@@ -2347,7 +2348,7 @@ hipError_t launch_gateup_tiles(const Shape &s, const LayerDev &L, const Scratch 
  * serves its four FMAs.
  *
  * Activation records (kMxRec bytes per slot, or per token, and 32-block) carry x in that
- * order as f16 (64 bytes; for Q4 rows lanes 4-7 hold x / 16), then d 2^24 (or the NaN that sends the chunk to the unscaled
+ * order as f16 (64 bytes; lanes 4-7 hold x / 16), then d 2^24 (or the NaN that sends the chunk to the unscaled
  * chains), ds, the half sums and d (16 bytes), then 16 zero bytes, which the lanes of A
  * outside their group read; the kernels stage those first 96 bytes of each record. Gate/up
  * writes the records of the activations it quantises, so the down products read them
@@ -3458,12 +3459,9 @@ static void launch_mx_shape(const MxArgs &a, int rows, int maxt, hipStream_t st)
 /* Other shapes of the same kernel measured at the 512-token prefill: 32-slot blocks of 16
  * waves (one per CU) 1.76 ms for gate/up, 64-row blocks of 4 waves (three per CU) 1.25,
  * against 1.24 for the wide blocks.
- * Staging buffers: the 8-slot blocks of 4 waves, and the 4-slot Q6_K down blocks, stage one
- * chunk at a time (half the LDS, so four blocks share a CU instead of two or three: the waves of
- * other blocks cover each block's copy); the others double-buffer. Measured at the 235B shape,
- * one buffer against two: Q6_K down 236 / 303 us at 4 slots per expert, 124 / 154 at 1 slot;
- * Q4_0 down 129 / 148 at 4 slots, 72.5 / 70.6 at 1 slot; the 4-slot gate/up blocks 297 / 287 at
- * 4 slots; the wide blocks 481 / 463 (Q6_K down) and 510 / 455 (gate/up) at 8 slots. */
+ * Staging buffers: the Q6_K gate/up blocks of 8 slots stage one chunk at a time (half the LDS, so
+ * four blocks share a CU: the waves of other blocks cover each block's copy), the others two or,
+ * 16-slot waves, two of weights and one of records. */
 template <int TYPE, int GU>
 static void launch_mx(const MxArgs &a, int rows, int maxt, MxShape shape, hipStream_t st)
 {
