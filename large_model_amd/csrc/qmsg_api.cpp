@@ -765,16 +765,19 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
     if (T == 0) return QMSG_OK;
     if (!d_x || ((uintptr_t)d_x & 15)) return fail(c, QMSG_E_INVALID, "qmsg_matmul_n: x must be 16-byte aligned");
     HIP_TRY(c, hipSetDevice(c->device));
-    /* The record buffer. Calls of fewer than kDenseQuantT rows can do without it (a captured call,
-     * or no memory: the row kernels), larger ones with the smaller pair records. */
+    /* The record buffer. Calls of fewer than kDenseQuantT rows can do without it (no memory: the row
+     * kernels), larger ones with the smaller pair records. A later, larger call replaces the buffer,
+     * so a graph must not hold it where it need not: captured calls of fewer than kDenseQuantT rows
+     * always take the row kernels, whatever the buffer holds. */
     bool mfma = T >= kDenseRecordT;
+    if (mfma && T < kDenseQuantT) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
+        mfma = cap == hipStreamCaptureStatusNone;
+    }
     if (mfma && c->dense_xqk_bytes < dense_record_bytes((size_t)T, (size_t)C)) {
         const size_t pairs = (size_t)T * (size_t)(C / 64) * kPairBytes;
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (T < kDenseQuantT) HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
-        int rc = cap == hipStreamCaptureStatusNone
-                     ? grow(c, &c->dense_xqk, &c->dense_xqk_bytes, dense_record_bytes((size_t)T, (size_t)C))
-                     : QMSG_E_NOMEM;
+        int rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, dense_record_bytes((size_t)T, (size_t)C));
         mfma = rc == QMSG_OK;
         if (rc == QMSG_E_NOMEM && T < kDenseQuantT) rc = QMSG_OK;
         else if (rc == QMSG_E_NOMEM) rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, pairs);

@@ -1,0 +1,150 @@
+/* Host side of the dense calls (csrc/qmsg_api.cpp) against a small stand-in for the HIP runtime and
+ * the launchers: which buffer each launch is given, and whether it outlives the graph that holds it.
+ * The stand-in keeps the runtime's rules the calls depend on: a failed call's error stays the
+ * thread's last error until hipGetLastError reads it, launchers return that error, and a
+ * synchronisation or free on a capturing stream fails.
+ *
+ *     dense_call_host SCENARIO        exit 0, or a line on stderr and exit 1 */
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "../include/qmsg.h"
+#include "../large_model_amd/csrc/qmsg_internal.h"
+
+namespace {
+
+std::set<void *> live;
+size_t malloc_limit = ~(size_t)0;      /* larger allocations fail */
+int mallocs = 0;
+hipError_t last = hipSuccess;
+bool capturing = false;
+
+hipError_t ret(hipError_t e)
+{
+    if (e != hipSuccess) last = e;
+    return e;
+}
+
+struct Launch {
+    bool exact, records;
+    int T, type;
+    uint8_t *xqk;
+};
+std::vector<Launch> launches;
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n)
+{
+    mallocs++;
+    if (n > malloc_limit) return ret(hipErrorOutOfMemory);
+    *p = malloc(64);                   /* addresses only */
+    live.insert(*p);
+    return hipSuccess;
+}
+/* freed blocks stay reserved, so that an address is never handed out twice */
+hipError_t hipFree(void *p) { live.erase(p); return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = malloc(n); return hipSuccess; }
+hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipGetLastError() { const hipError_t e = last; last = hipSuccess; return e; }
+const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
+hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
+hipError_t hipGetSymbolAddress(void **p, const void *s) { *p = (void *)s; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)8; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s)
+{
+    *s = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipMemset(void *, int, size_t) { return hipSuccess; }
+hipError_t hipMemcpy(void *, const void *, size_t, hipMemcpyKind) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void *, const void *, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+}
+
+namespace qmsg {
+thread_local const LaunchTimer *g_launch_timer = nullptr;
+hipError_t launch_dense(const DenseArgs &a, int type, uint8_t *xqk, uint64_t, bool *records, hipStream_t)
+{
+    launches.push_back({ false, records != nullptr, a.T, type, xqk });
+    return hipGetLastError();
+}
+hipError_t launch_dense_exact(const DenseArgs &a, int type, hipStream_t)
+{
+    launches.push_back({ true, false, a.T, type, nullptr });
+    return hipGetLastError();
+}
+}  // namespace qmsg
+
+#define CHECK(c)                                                                     \
+    do {                                                                             \
+        if (!(c)) { fprintf(stderr, "line %d: %s (%s)\n", __LINE__, #c, qmsg_last_error(ctx)); exit(1); } \
+    } while (0)
+
+static qmsg_ctx *ctx;
+
+static int mat(int type, int64_t rows, int64_t cols)
+{
+    static uint8_t data[16];
+    const uint64_t rb = type == QMSG_T_Q4_0 ? (uint64_t)cols / 32 * 18
+                        : type == QMSG_T_Q8_0 ? (uint64_t)cols / 32 * 34
+                        : type == QMSG_T_Q6_K ? (uint64_t)cols / 256 * 210 : (uint64_t)cols * 4;
+    const qmsg_mat m = { type, rows, cols, rb, data };
+    int id = -1;
+    CHECK(qmsg_mat_upload(ctx, &m, &id) == QMSG_OK);
+    return id;
+}
+
+static int call(int id, int T)
+{
+    float *const x = (float *)4096;
+    float *const y[1] = { (float *)8192 };
+    return qmsg_matmul_n_device(ctx, &id, 1, x, T, y);
+}
+
+/* the buffers that the launches recorded so far would use when replayed */
+static bool launches_safe(size_t first, size_t end)
+{
+    for (size_t i = first; i < end; i++) {
+        const Launch &l = launches[i];
+        const bool uses = !l.exact && (l.records || l.T >= qmsg::kDenseQuantT);
+        if (uses && l.xqk && !live.count(l.xqk)) return false;
+    }
+    return true;
+}
+
+/* a captured call of 5-7 rows on a large matrix, after a call that left the buffer large enough */
+static void capture_small()
+{
+    const int big = mat(QMSG_T_Q4_0, 8192, 4096);
+    for (int T = 5; T < qmsg::kDenseQuantT; T++) {
+        CHECK(call(big, 8 * T) == QMSG_OK);
+        capturing = true;
+        const size_t n = launches.size();
+        CHECK(call(big, T) == QMSG_OK);
+        capturing = false;
+        CHECK(launches.size() == n + 1 && !launches[n].records);
+        CHECK(call(big, 64 * T) == QMSG_OK);        /* replaces the buffer */
+        CHECK(launches_safe(n, n + 1));
+        CHECK(call(big, T) == QMSG_OK && launches.back().records);
+    }
+}
+
+int main(int argc, char **argv)
+{
+    const qmsg_cfg cfg = { 256, 16, 4, 128 };
+    if (argc != 2 || qmsg_create(&ctx, 0, &cfg, 1, 1) != QMSG_OK) return 2;
+    const std::string s = argv[1];
+    if (s == "capture_small") capture_small();
+    else return 2;
+    qmsg_destroy(ctx);
+    return 0;
+}
