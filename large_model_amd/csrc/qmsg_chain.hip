@@ -216,12 +216,12 @@ __device__ __forceinline__ void ch_vals(const ChRaw<TYPE> &r, int b, float (&v)[
 template <int TYPE>
 size_t ch_lds(int NC) { return 4 * (size_t)ChFmt<TYPE>::WAVE + 2 * (size_t)(16 * NC * ChFmt<TYPE>::XS) * 4; }
 template <int TYPE>
-size_t ch_lds_res(int T, int C) { return 4 * (size_t)ChFmt<TYPE>::WAVE + (size_t)T * (C + 4) * 4; }
+size_t ch_lds_res(int T, int C) { return 4 * (size_t)ChFmt<TYPE>::WAVE + chain_rows_lds(T, C); }
 
 /* The chains of a wave's 16 rows over nblk 32-blocks: row i (clamped to rows - 1) at wb + i * rb, wb
  * wave-uniform; acc[n] takes row 4 (lane / 16) + v, input row 16 n + lane % 16. Not RES: thread t
- * stages the input rows xr[n] for t / 16 + 16 n at xsm. RES: the block has staged input rows of
- * nblk * 32 + 4 floats, and xl is the lane's row there. Every wave passes the same barriers; all
+ * stages the input rows xr[n] for t / 16 + 16 n at xsm. RES: the block has staged its input rows
+ * (chain_rows_lds), and xl is the lane's row there. Every wave passes the same barriers; all
  * LDS reads are done at the end except other waves' (of their own rows, or of RES inputs). */
 template <int TYPE, int NC, bool RES>
 __device__ __forceinline__ void chain_tile(uint8_t *wsm, float *xsm, const uint8_t *wb, uint32_t rb, int rows,
@@ -291,8 +291,8 @@ __device__ __forceinline__ void chain_tile(uint8_t *wsm, float *xsm, const uint8
         for (int n = 0; n < NC; n++)
 #pragma unroll
             for (int q = 0; q < 2; q++)
-                b[n][q] = *(const f32x4 *)((RES ? xl + 32 * (XB * st + k)
-                                                : xsm + (st & 1) * XBUF + (16 * n + i) * F::XS + 32 * k) + 8 * g + 4 * q);
+                b[n][q] = *(const f32x4 *)(RES ? xl + chain_row_read(XB * st + k, g, q)
+                                               : xsm + (st & 1) * XBUF + (16 * n + i) * F::XS + 32 * k + 8 * g + 4 * q);
     };
     float a[8];
 #pragma unroll
@@ -394,7 +394,7 @@ __device__ __forceinline__ void chain_rows_of(uint8_t *smem, const uint8_t *wb, 
     chain_tile<TYPE, NC, RES>(wsm, xsm, wb, (uint32_t)rb, rows, xr, xl, nblk, acc);
 }
 
-/* Input rows staged whole, as [row][block][g][8] at C + 4 floats per row; src(r) is row r. */
+/* Input rows staged whole, as [row][block][g][8] at chain_row_floats(C) per row; src(r) is row r. */
 template <class Src>
 __device__ __forceinline__ void chain_stage(float *xsm, int rows, int C, Src src)
 {
@@ -402,7 +402,7 @@ __device__ __forceinline__ void chain_stage(float *xsm, int rows, int C, Src src
     for (int k = threadIdx.x; k < rows * q4; k += 256) {
         const int r = k / q4, q = k - r * q4;
         const f32x4 v = *(const f32x4 *)(src(r) + 4 * q);
-        float *d = xsm + r * (C + 4) + 32 * (q >> 3) + (q & 7);
+        float *d = xsm + r * chain_row_floats(C) + 32 * (q >> 3) + (q & 7);
 #pragma unroll
         for (int j = 0; j < 4; j++) d[8 * j] = v[j];
     }
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256) void chain_rows_kernel(ChainArgs a)
     if constexpr (RES) {
         float *xsm = (float *)(chsm + 4 * ChFmt<TYPE>::WAVE);
         chain_stage(xsm, ns, a.cols, src);
-        xl = xsm + min(lane & 15, ns - 1) * (a.cols + 4);
+        xl = xsm + min(lane & 15, ns - 1) * chain_row_floats(a.cols);
         xr[0] = nullptr;
     } else {
 #pragma unroll
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(256) void chain_dense_kernel(DenseArgs a)
     if constexpr (RES) {
         float *xsm = (float *)(chsm + 4 * ChFmt<TYPE>::WAVE);
         chain_stage(xsm, nt, a.C, src);
-        xl = xsm + min(lane & 15, nt - 1) * (a.C + 4);
+        xl = xsm + min(lane & 15, nt - 1) * chain_row_floats(a.C);
         xr[0] = nullptr;
     } else {
 #pragma unroll

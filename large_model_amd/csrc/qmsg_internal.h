@@ -248,6 +248,13 @@ struct ChainRows {
     float *y;
     int y_stride;
 };
+/* Input rows the chain kernels stage whole in LDS: C + 4 floats a row, blocks as [g][8]. A lane
+ * reads its group's words of the block after the one it multiplies, so after the last block those
+ * of block C / 32, which it does not use: of the next row, or past the last row the 28 floats that
+ * chain_rows_lds adds. */
+__host__ __device__ constexpr int chain_row_floats(int C) { return C + 4; }
+__host__ __device__ constexpr int chain_row_read(int block, int group, int quad) { return 32 * block + 8 * group + 4 * quad; }
+constexpr size_t chain_rows_lds(int rows, int C) { return ((size_t)rows * (size_t)chain_row_floats(C) + 28) * 4; }
 hipError_t launch_chain_rows(const char *name, const ChainRows &m, const ChainRows *up, const Scratch &S, int T,
                              int max_tiles, float *gu, hipStream_t st);
 hipError_t launch_block_dots(const uint8_t *base, int type, uint64_t rb, uint64_t eb, int n, const int32_t *expert,

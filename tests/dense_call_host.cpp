@@ -138,12 +138,24 @@ static void capture_small()
     }
 }
 
+/* the chain kernels' reads of input rows staged whole, the block read ahead included, stay inside
+ * the LDS their launch asks for */
+static void chain_lds()
+{
+    for (int T = 1; T <= 16; T++)
+        for (int C = 32; T * C <= 16384; C += 32) {
+            const int end = (T - 1) * qmsg::chain_row_floats(C) + qmsg::chain_row_read(C / 32, 3, 1) + 4;
+            CHECK((size_t)end * 4 <= qmsg::chain_rows_lds(T, C));
+        }
+}
+
 int main(int argc, char **argv)
 {
     const qmsg_cfg cfg = { 256, 16, 4, 128 };
     if (argc != 2 || qmsg_create(&ctx, 0, &cfg, 1, 1) != QMSG_OK) return 2;
     const std::string s = argv[1];
     if (s == "capture_small") capture_small();
+    else if (s == "chain_lds") chain_lds();
     else return 2;
     qmsg_destroy(ctx);
     return 0;

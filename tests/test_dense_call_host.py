@@ -1,5 +1,6 @@
 """The host side of the dense calls on a stand-in for the HIP runtime (tests/dense_call_host.cpp, CPU):
-the record buffer under graph capture, when it grows and when it cannot be allocated."""
+the record buffer under graph capture, when it grows and when it cannot be allocated; and the LDS that the
+fp32-chain kernels ask for against what they read."""
 import os
 import shutil
 import subprocess
@@ -27,5 +28,13 @@ def exe(tmp_path_factory):
 
 @pytest.mark.parametrize("scenario", ["capture_small"])
 def test_record_buffer(exe, scenario):
+    run(exe, scenario)
+
+
+def test_chain_rows_lds(exe):
+    run(exe, "chain_lds")
+
+
+def run(exe, scenario):
     r = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr[-2000:]
