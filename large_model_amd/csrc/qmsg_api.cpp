@@ -168,17 +168,25 @@ static int fail(qmsg_ctx *c, int code, const char *fmt, ...)
     return code;
 }
 
+/* A failed runtime call's error also stays the thread's last error, which the next launch would
+ * report as its own: it is cleared where the failure is returned or absorbed. */
 #define HIP_TRY(c, call)                                                                               \
     do {                                                                                               \
         hipError_t e_ = (call);                                                                        \
-        if (e_ != hipSuccess) return fail((c), QMSG_E_DEVICE, "%s: %s", #call, hipGetErrorString(e_)); \
+        if (e_ != hipSuccess) {                                                                        \
+            (void)hipGetLastError();                                                                   \
+            return fail((c), QMSG_E_DEVICE, "%s: %s", #call, hipGetErrorString(e_));                   \
+        }                                                                                              \
     } while (0)
 
 static int dev_alloc(qmsg_ctx *c, void **p, size_t bytes, std::vector<void *> &list)
 {
     /* 256 bytes of tail padding: kernels may read one aligned word past a tensor's end. */
     hipError_t e = hipMalloc(p, bytes + 256);
-    if (e != hipSuccess) return fail(c, QMSG_E_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(c, QMSG_E_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    }
     list.push_back(*p);
     return QMSG_OK;
 }

@@ -138,6 +138,32 @@ static void capture_small()
     }
 }
 
+/* no memory for the record buffer: 5-7 rows fall to the row kernels, 8 and more to the smaller pair
+ * records, and with none for those either the call says so; nothing of it reaches the next call */
+static void no_memory()
+{
+    const int C = 4096, big = mat(QMSG_T_Q4_0, 8192, C), f32 = mat(QMSG_T_F32, 8, C);
+    malloc_limit = 4096;
+    for (int T = 5; T < qmsg::kDenseQuantT; T++) {
+        CHECK(call(big, T) == QMSG_OK && !launches.back().records);
+        CHECK(call(f32, 1) == QMSG_OK);
+    }
+    CHECK(call(big, 16) == QMSG_E_NOMEM);
+    CHECK(call(f32, 1) == QMSG_OK);
+    malloc_limit = 16 * (C / 64) * qmsg::kPairBytes + 256;
+    CHECK(call(big, 16) == QMSG_OK && !launches.back().records && launches.back().xqk);
+    CHECK(call(big, 16) == QMSG_OK && !launches.back().records);
+    CHECK(qmsg_device_alloc(ctx, (size_t)1 << 40) == nullptr);
+    CHECK(call(f32, 1) == QMSG_OK);
+    malloc_limit = ~(size_t)0;
+    CHECK(call(big, 16) == QMSG_OK && launches.back().records);
+    /* a captured call that would have to replace the buffer is refused, the next one runs */
+    capturing = true;
+    CHECK(call(big, 512) == QMSG_E_DEVICE);
+    capturing = false;
+    CHECK(call(f32, 1) == QMSG_OK);
+}
+
 /* the chain kernels' reads of input rows staged whole, the block read ahead included, stay inside
  * the LDS their launch asks for */
 static void chain_lds()
@@ -155,6 +181,7 @@ int main(int argc, char **argv)
     if (argc != 2 || qmsg_create(&ctx, 0, &cfg, 1, 1) != QMSG_OK) return 2;
     const std::string s = argv[1];
     if (s == "capture_small") capture_small();
+    else if (s == "no_memory") no_memory();
     else if (s == "chain_lds") chain_lds();
     else return 2;
     qmsg_destroy(ctx);

@@ -26,7 +26,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("scenario", ["capture_small"])
+@pytest.mark.parametrize("scenario", ["capture_small", "no_memory"])
 def test_record_buffer(exe, scenario):
     run(exe, scenario)
 

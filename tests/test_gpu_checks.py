@@ -186,3 +186,22 @@ def test_arguments_and_repeated_calls(q):
             l = i % 2
             out = ctx.moe(l, x)
             assert np.array_equal(out.view(np.uint32), refs[l].moe(x).view(np.uint32)), i
+
+
+def test_call_after_failed_allocation():
+    """An allocation no device can hold is refused; its error does not reach the next calls."""
+    from large_model_amd import qmsg
+    E, X, K, F, cols, rows = 256, 16, 4, 128, 256, 64
+    print("[case] calls after a failed allocation", flush=True)
+    w, x = orc.synth_mat(orc.T_Q4_0, rows, cols, 9), orc.make_input(cols, 3, 10)
+    with qmsg.Context(E, X, K, F, max_tokens=3) as ctx:
+        ctx.synth(0, 11)
+        i = ctx.mat_upload(orc.T_Q4_0, w, rows, cols)
+        with pytest.raises(qmsg.QmsgError):
+            ctx.device_alloc(1 << 50)
+        y = ctx.matmul_n([i], x)[0]
+        with pytest.raises(qmsg.QmsgError):
+            ctx.device_alloc(1 << 50)
+        out = ctx.moe(0, orc.make_input(E, 3, 11))
+    assert np.array_equal(y.view(np.uint32), orc.matmul_q8(orc.T_Q4_0, w, rows, cols, x).view(np.uint32))
+    assert np.array_equal(out.view(np.uint32), orc.Layer(E, X, K, F, 11).moe(orc.make_input(E, 3, 11)).view(np.uint32))
