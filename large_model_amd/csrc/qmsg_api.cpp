@@ -773,24 +773,6 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
     if (T == 0) return QMSG_OK;
     if (!d_x || ((uintptr_t)d_x & 15)) return fail(c, QMSG_E_INVALID, "qmsg_matmul_n: x must be 16-byte aligned");
     HIP_TRY(c, hipSetDevice(c->device));
-    /* The record buffer. Calls of fewer than kDenseQuantT rows can do without it (no memory: the row
-     * kernels), larger ones with the smaller pair records. A later, larger call replaces the buffer,
-     * so a graph must not hold it where it need not: captured calls of fewer than kDenseQuantT rows
-     * always take the row kernels, whatever the buffer holds. */
-    bool mfma = T >= kDenseRecordT;
-    if (mfma && T < kDenseQuantT) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
-        mfma = cap == hipStreamCaptureStatusNone;
-    }
-    if (mfma && c->dense_xqk_bytes < dense_record_bytes((size_t)T, (size_t)C)) {
-        const size_t pairs = (size_t)T * (size_t)(C / 64) * kPairBytes;
-        int rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, dense_record_bytes((size_t)T, (size_t)C));
-        mfma = rc == QMSG_OK;
-        if (rc == QMSG_E_NOMEM && T < kDenseQuantT) rc = QMSG_OK;
-        else if (rc == QMSG_E_NOMEM) rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, pairs);
-        if (rc) return rc;
-    }
     /* qms_matmul_n's choice for the whole call (src/quant.c:131-141): the fast loop, or
      * matmul_exact for every matrix when --exact is set or one of them is F16 / Q8_0 */
     bool exact = c->path == QMSG_PATH_FP32;
@@ -801,9 +783,14 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
     if (exact && C * 4 > 160 * 1024)
         return fail(c, QMSG_E_UNSUPPORTED, "qmsg_matmul_n: fp32-chain rows above %d columns", 160 * 1024 / 4);
     /* launches of up to kDenseMats matrices of one type, in argument order */
+    struct Group {
+        DenseArgs a;
+        int type;
+    };
+    std::vector<Group> groups;
     std::vector<bool> done((size_t)nW, false);
-    const uint64_t epoch = next_epoch();
-    bool records = false;
+    bool mfma = false;
+    size_t pairs = 0;
     for (int i = 0; i < nW; i++) {
         if (done[(size_t)i]) continue;
         const int type = c->mats[(size_t)ids[i]].type;
@@ -821,8 +808,33 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
             a.nm++;
             done[(size_t)j] = true;
         }
-        if (exact) LAUNCH(c, "dense", launch_dense_exact(a, type, c->stream));
-        else LAUNCH(c, "dense", launch_dense(a, type, (uint8_t *)c->dense_xqk, epoch, mfma ? &records : nullptr, c->stream));
+        groups.push_back({ a, type });
+        if (exact) continue;
+        mfma = mfma || dense_mx_takes(a, type);
+        if (dense_pairs_taken(type, (int)C, T)) pairs = (size_t)T * (size_t)(C / 64) * kPairBytes;
+    }
+    /* The record buffer, where a launch of this call reads it: the MFMA records, or the smaller pair
+     * records of the row kernels, which take over without memory for the others (of fewer than
+     * kDenseQuantT rows they read none). A later, larger call replaces the buffer, so a graph must
+     * not hold it where it need not: captured calls of fewer than kDenseQuantT rows always take the
+     * row kernels, larger ones what the buffer already holds. */
+    const size_t recs = dense_record_bytes((size_t)T, (size_t)C);
+    if (mfma && (T < kDenseQuantT || c->dense_xqk_bytes < recs)) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
+        if (cap != hipStreamCaptureStatusNone && c->dense_xqk_bytes >= pairs) mfma = false;
+    }
+    int rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, mfma ? recs : pairs);
+    if (rc == QMSG_E_NOMEM && mfma) {
+        mfma = false;
+        rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, pairs);
+    }
+    if (rc) return rc;
+    const uint64_t epoch = next_epoch();
+    bool records = false;
+    for (const Group &g : groups) {
+        if (exact) LAUNCH(c, "dense", launch_dense_exact(g.a, g.type, c->stream));
+        else LAUNCH(c, "dense", launch_dense(g.a, g.type, (uint8_t *)c->dense_xqk, epoch, mfma ? &records : nullptr, c->stream));
     }
     return QMSG_OK;
 }

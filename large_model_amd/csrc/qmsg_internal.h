@@ -134,8 +134,26 @@ struct DenseArgs {
 /* Batches of at least this many rows are quantised once by a separate launch; smaller ones
  * inside every dense block. */
 constexpr int kDenseQuantT = 8;
-/* Batches from which a dense call may need the record buffer (its MFMA kernels: from 5 rows). */
-constexpr int kDenseRecordT = 5;
+/* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
+ * read (Q6_K: 4-byte aligned), a block's rows in each matrix, and enough tokens. us per launch
+ * pair with the records at the 235B / 30B shapes, MFMA / row kernels: Q4_0 58 / 43 and 35 / 21 at
+ * 4 tokens, about 59 / 72 and 35 / 33 at 6, 63 / 134 at 16; Q6_K 108 / 85 and 59 / 36 at 4, 112 /
+ * 137 and 60 / 49 at 6, 64 / 109 (30B) at 16, where the row kernels take another pass. */
+inline bool dense_mx_takes(const DenseArgs &a, int type)
+{
+    if ((type != 2 && type != 3 && type != 14) || a.C % 256 || (type == 14 && a.rb % 4) || a.T > 4 * 65535) return false;
+    long rows = 0;
+    for (int i = 0; i < a.nm; i++) {
+        if (a.m[i].rows < 128) return false;
+        rows += a.m[i].rows;
+    }
+    return a.T > 8 || (a.T > 4 && rows * a.C >= 1l << 24);
+}
+
+/* Widths of the chunked row kernels (others: the direct-read kernel), and whether those read pair
+ * records from the record buffer (else every block quantises the rows it reads). */
+inline bool dense_chunked(int type, int C) { return type == 14 ? C % 2048 == 0 : C % 256 == 0; }
+inline bool dense_pairs_taken(int type, int C, int T) { return type != 0 && dense_chunked(type, C) && T >= kDenseQuantT; }
 
 /* Launchers (qmsg_kernels.hip). Each returns hipSuccess or the launch error. */
 hipError_t launch_route(const Shape &s, const LayerDev &L, const Scratch &S, const float *xn, int T,
@@ -228,10 +246,11 @@ hipError_t launch_exp(const double *x, int n, double *out, hipStream_t st);
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
 /* p[0 .. n-1] = v (a kernel, not a memset node: safe inside a captured graph). */
 hipError_t launch_call_reset(const Scratch &S, hipStream_t st);
-/* The dense rows kernel; for T >= kDenseQuantT (MFMA kernels: kDenseRecordT) the input records are formed first into xqk
- * (dense_record_bytes), whose flag word takes epoch (unique per call) when one is outside the
- * MFMA kernels' scaled range. *records: xqk holds the MFMA records of this call's rows (formed by an
- * earlier launch of the call); updated. NULL: no MFMA kernels (xqk smaller or NULL). */
+/* The dense rows kernel. Where dense_mx_takes or dense_pairs_taken the input records are formed first
+ * into xqk: MFMA records (dense_record_bytes), whose flag word takes epoch (unique per call) when
+ * one is outside the MFMA kernels' scaled range, or pair records. *records: xqk holds the MFMA records
+ * of this call's rows (formed by an earlier launch of the call); updated. NULL: no MFMA kernels (xqk
+ * smaller or NULL). */
 inline size_t dense_record_bytes(size_t T, size_t C) { return 256 + T * (C / 32) * kMxRec; }
 hipError_t launch_dense(const DenseArgs &a, int type, uint8_t *xqk, uint64_t epoch, bool *records, hipStream_t st);
 /* matmul_exact for every matrix of a call (--exact, or an F16 / Q8_0 matrix in the call). */

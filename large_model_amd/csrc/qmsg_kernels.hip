@@ -3635,22 +3635,6 @@ static void launch_dense_mx_type(const MxArgs &a, hipStream_t st)
     }
 }
 
-/* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
- * read (Q6_K: 4-byte aligned), a block's rows in each matrix, and enough tokens. us per launch
- * pair with the records at the 235B / 30B shapes, MFMA / row kernels: Q4_0 58 / 43 and 35 / 21 at
- * 4 tokens, about 59 / 72 and 35 / 33 at 6, 63 / 134 at 16; Q6_K 108 / 85 and 59 / 36 at 4, 112 /
- * 137 and 60 / 49 at 6, 64 / 109 (30B) at 16, where the row kernels take another pass. */
-static bool dense_mx_takes(const DenseArgs &a, int type)
-{
-    if ((type != 2 && type != 3 && type != 14) || a.C % 256 || (type == 14 && a.rb % 4) || a.T > 4 * 65535) return false;
-    long rows = 0;
-    for (int i = 0; i < a.nm; i++) {
-        if (a.m[i].rows < 128) return false;
-        rows += a.m[i].rows;
-    }
-    return a.T > 8 || (a.T > 4 && rows * a.C >= 1l << 24);
-}
-
 static hipError_t launch_dense_mx(const DenseArgs &d, int type, uint8_t *buf, uint64_t epoch, bool records,
                                   hipStream_t st)
 {
@@ -4449,7 +4433,7 @@ hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t 
         *records = true;
         return launch_dense_mx(a, type, xqk, epoch, have, st);
     }
-    if (type != 0 && (type == 14 ? nb % 64 != 0 : nb % 8 != 0)) {
+    if (type != 0 && !dense_chunked(type, a.C)) {
         /* widths the chunked kernels do not take: one direct-read pass per NT tokens */
         const int NT = dense_any_nt(type, a.T, nb);
         if (!NT) return hipErrorInvalidValue;
@@ -4483,7 +4467,7 @@ hipError_t launch_dense(const DenseArgs &args, int type, uint8_t *xqk, uint64_t 
         return hipGetLastError();
     }
     a.xqk = nullptr;
-    if (a.T >= kDenseQuantT && xqk) {
+    if (dense_pairs_taken(type, a.C, a.T) && xqk) {
         QLAUNCH("dquant", dense_quant_kernel, dim3((a.T * nb + 255) / 256), dim3(256), 0, st, a.x, a.C, a.T, xqk);
         a.xqk = xqk;
         if (records) *records = false;        /* the pair records took their place */

@@ -164,6 +164,37 @@ static void no_memory()
     CHECK(call(f32, 1) == QMSG_OK);
 }
 
+/* calls whose launches read no record buffer allocate none: fp32 chains, F32 rows, widths of the
+ * direct-read kernel, and at 5-7 rows matrices too small for the MFMA kernels; 8 and more rows on
+ * the row kernels allocate the pair records only */
+static void no_buffer()
+{
+    const int q8 = mat(QMSG_T_Q8_0, 8192, 4096), f32 = mat(QMSG_T_F32, 8192, 4096), big = mat(QMSG_T_Q4_0, 8192, 4096);
+    const int off = mat(QMSG_T_Q4_0, 8192, 4128), small = mat(QMSG_T_Q4_0, 256, 256), few = mat(QMSG_T_Q4_0, 64, 4096);
+    const int n = mallocs;
+    for (int T : { 1, 4, 5, 7, 8, 64 }) {
+        CHECK(call(q8, T) == QMSG_OK && call(f32, T) == QMSG_OK && call(off, T) == QMSG_OK);
+        if (T < qmsg::kDenseQuantT) CHECK(call(small, T) == QMSG_OK && call(few, T) == QMSG_OK);
+        CHECK(qmsg_set_path(ctx, QMSG_PATH_FP32) == QMSG_OK);
+        CHECK(call(big, T) == QMSG_OK);
+        CHECK(qmsg_set_path(ctx, QMSG_PATH_AUTO) == QMSG_OK);
+    }
+    CHECK(mallocs == n);
+    malloc_limit = 64 * (4096 / 64) * qmsg::kPairBytes + 256;
+    CHECK(call(few, 64) == QMSG_OK && mallocs == n + 1);
+}
+
+/* a captured call that pair records suffice for uses those there are */
+static void capture_pairs()
+{
+    const int big = mat(QMSG_T_Q4_0, 8192, 4096);
+    malloc_limit = 16 * (4096 / 64) * qmsg::kPairBytes + 256;
+    CHECK(call(big, 16) == QMSG_OK && !launches.back().records);
+    capturing = true;
+    CHECK(call(big, 16) == QMSG_OK && !launches.back().records && live.count(launches.back().xqk));
+    capturing = false;
+}
+
 /* the chain kernels' reads of input rows staged whole, the block read ahead included, stay inside
  * the LDS their launch asks for */
 static void chain_lds()
@@ -182,6 +213,8 @@ int main(int argc, char **argv)
     const std::string s = argv[1];
     if (s == "capture_small") capture_small();
     else if (s == "no_memory") no_memory();
+    else if (s == "no_buffer") no_buffer();
+    else if (s == "capture_pairs") capture_pairs();
     else if (s == "chain_lds") chain_lds();
     else return 2;
     qmsg_destroy(ctx);
