@@ -135,13 +135,15 @@ struct DenseArgs {
  * inside every dense block. */
 constexpr int kDenseQuantT = 8;
 /* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
- * read (Q6_K: 4-byte aligned), a block's rows in each matrix, and enough tokens. us per launch
+ * read (Q6_K: 4-byte aligned), a block's rows in each matrix and their bytes in the 31 bits of its
+ * offsets (128 rows of under 2^24 bytes), and enough tokens. us per launch
  * pair with the records at the 235B / 30B shapes, MFMA / row kernels: Q4_0 58 / 43 and 35 / 21 at
  * 4 tokens, about 59 / 72 and 35 / 33 at 6, 63 / 134 at 16; Q6_K 108 / 85 and 59 / 36 at 4, 112 /
  * 137 and 60 / 49 at 6, 64 / 109 (30B) at 16, where the row kernels take another pass. */
 inline bool dense_mx_takes(const DenseArgs &a, int type)
 {
-    if ((type != 2 && type != 3 && type != 14) || a.C % 256 || (type == 14 && a.rb % 4) || a.T > 4 * 65535) return false;
+    if ((type != 2 && type != 3 && type != 14) || a.C % 256 || (type == 14 && a.rb % 4) || a.rb >= 1u << 24 || a.T > 4 * 65535)
+        return false;
     long rows = 0;
     for (int i = 0; i < a.nm; i++) {
         if (a.m[i].rows < 128) return false;

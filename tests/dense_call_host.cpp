@@ -195,6 +195,23 @@ static void capture_pairs()
     capturing = false;
 }
 
+/* rows so long that a block's byte offsets (32 bits, the top one a flag) would not hold them stay off
+ * the MFMA kernels */
+static void wide_rows()
+{
+    for (int type : { QMSG_T_Q4_0, QMSG_T_Q4_1, QMSG_T_Q6_K })
+        for (int64_t C : { (int64_t)4096, (int64_t)1 << 22, (int64_t)1 << 24, (int64_t)1 << 26, (int64_t)1 << 30 }) {
+            qmsg::DenseArgs a{};
+            a.rb = (uint64_t)(type == QMSG_T_Q4_0 ? C / 32 * 18 : type == QMSG_T_Q4_1 ? C / 32 * 20 : C / 256 * 210);
+            a.C = (int)C;
+            a.T = 16;
+            a.nm = 1;
+            a.m[0].rows = 128;
+            CHECK(!qmsg::dense_mx_takes(a, type) || 128 * a.rb < (uint64_t)1 << 31);
+            CHECK(C > 4096 || qmsg::dense_mx_takes(a, type));
+        }
+}
+
 /* the chain kernels' reads of input rows staged whole, the block read ahead included, stay inside
  * the LDS their launch asks for */
 static void chain_lds()
@@ -215,6 +232,7 @@ int main(int argc, char **argv)
     else if (s == "no_memory") no_memory();
     else if (s == "no_buffer") no_buffer();
     else if (s == "capture_pairs") capture_pairs();
+    else if (s == "wide_rows") wide_rows();
     else if (s == "chain_lds") chain_lds();
     else return 2;
     qmsg_destroy(ctx);

@@ -1,6 +1,6 @@
 """The host side of the dense calls on a stand-in for the HIP runtime (tests/dense_call_host.cpp, CPU):
 the record buffer under graph capture, when it grows and when it cannot be allocated; and the LDS that the
-fp32-chain kernels ask for against what they read."""
+fp32-chain kernels ask for against what they read, and the row lengths the MFMA kernels address."""
 import os
 import shutil
 import subprocess
@@ -31,8 +31,9 @@ def test_record_buffer(exe, scenario):
     run(exe, scenario)
 
 
-def test_chain_rows_lds(exe):
-    run(exe, "chain_lds")
+@pytest.mark.parametrize("scenario", ["chain_lds", "wide_rows"])
+def test_kernel_limits(exe, scenario):
+    run(exe, scenario)
 
 
 def run(exe, scenario):
