@@ -426,8 +426,9 @@ template <int TYPE, int NC, bool PAIR, bool RES>
 __global__ __launch_bounds__(256) void chain_rows_kernel(ChainArgs a)
 {
     extern __shared__ __align__(16) uint8_t chsm[];
-    if ((int)blockIdx.y >= a.S.meta[1]) return;
-    const int4 tl = a.S.tiles[blockIdx.y];
+    const int tile = (int)(blockIdx.z * gridDim.y + blockIdx.y);
+    if (tile >= a.S.meta[1]) return;
+    const int4 tl = a.S.tiles[tile];
     const int e = tl.x, s0 = tl.y, ns = tl.z - tl.y;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int R0 = (int)blockIdx.x * (PAIR ? 32 : 64);
@@ -541,6 +542,13 @@ bool with_type(int type, F f)
     }
 }
 
+/* Tiles over y and z: a grid's y ends at 65535, and 32,768 tokens of 64 experts make more. */
+dim3 chain_grid(int blocks, int tiles)
+{
+    const int ty = tiles < 32768 ? tiles : 32768;
+    return dim3(blocks, ty, (tiles + ty - 1) / ty);
+}
+
 }  // namespace
 
 hipError_t launch_chain_rows(const char *name, const ChainRows &m, const ChainRows *up, const Scratch &S, int T,
@@ -564,7 +572,7 @@ hipError_t launch_chain_rows(const char *name, const ChainRows &m, const ChainRo
     /* an expert's slots are distinct tokens: up to 16 tokens every slot tile fits one
      * instruction's columns, and its input rows LDS where T of them do */
     const bool res = (size_t)T * m.cols <= kChResFloats && T <= 16;
-    const dim3 grid((m.rows + (up ? 31 : 63)) / (up ? 32 : 64), max_tiles), block(256);
+    const dim3 grid = chain_grid((m.rows + (up ? 31 : 63)) / (up ? 32 : 64), max_tiles), block(256);
     const bool ok = with_type(m.type, [&](auto ty) {
         constexpr int TY = decltype(ty)::value;
         /* LDS of the inputs whole, or of stages; gate/up's results take less than either */
@@ -591,14 +599,14 @@ hipError_t launch_dense_exact(const DenseArgs &args, int type, hipStream_t st)
         a.m[i].first_block = nblk;
         nblk += (a.m[i].rows + kChRows - 1) / kChRows;
     }
-    const int tiles = (a.T + 31) / 32, ty = tiles < 32768 ? tiles : 32768, tz = (tiles + ty - 1) / ty;
+    const dim3 grid = chain_grid(nblk, (a.T + 31) / 32);
     const bool ok = with_type(type, [&](auto tag) {
         constexpr int TY = decltype(tag)::value;
         const size_t whole = ch_lds_res<TY>(a.T, a.C);
         if (a.T <= 16 && (size_t)a.T * a.C <= kChResFloats)
             QLAUNCH("dense", (chain_dense_kernel<TY, 1, true>), dim3(nblk), dim3(256), whole, st, a);
         else if (a.T <= 16) QLAUNCH("dense", (chain_dense_kernel<TY, 1, false>), dim3(nblk), dim3(256), ch_lds<TY>(1), st, a);
-        else QLAUNCH("dense", (chain_dense_kernel<TY, 2, false>), dim3(nblk, ty, tz), dim3(256), ch_lds<TY>(2), st, a);
+        else QLAUNCH("dense", (chain_dense_kernel<TY, 2, false>), grid, dim3(256), ch_lds<TY>(2), st, a);
     });
     return ok ? hipGetLastError() : hipErrorInvalidValue;
 }

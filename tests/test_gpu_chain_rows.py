@@ -67,3 +67,18 @@ def test_chain_layer(q, T, types):
         ctx.upload(0, L.router, (types[0], L.gate), (types[1], L.up), (types[2], L.down))
         out = ctx.moe(0, x)
     assert np.array_equal(bits(out), bits(L.moe(x)))
+
+
+def test_chain_layer_many_tiles():
+    """More slot tiles than a grid's y takes (65535): one large call against the same tokens in parts."""
+    E, X, K, F, T = 32, 64, 64, 32, 33000
+    print(f"[case] chain layer {T} tokens x {K} experts", flush=True)
+    from large_model_amd import qmsg
+    L = et.typed_layer(E, X, K, F, (orc.T_Q8_0,) * 3, 62)
+    x = orc.make_input(E, T, 63)
+    with qmsg.Context(E, X, K, F, max_tokens=T) as ctx:
+        ctx.upload(0, L.router, *((orc.T_Q8_0, w) for w in (L.gate, L.up, L.down)))
+        out = ctx.moe(0, x)
+        parts = np.concatenate([ctx.moe(0, x[i:i + 11000]) for i in range(0, T, 11000)])
+    assert np.array_equal(bits(out), bits(parts))
+    assert np.array_equal(bits(out[-8:]), bits(L.moe(x[-8:])))
