@@ -136,10 +136,13 @@ struct DenseArgs {
 constexpr int kDenseQuantT = 8;
 /* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
  * read (Q6_K: 4-byte aligned), a block's rows in each matrix and their bytes in the 31 bits of its
- * offsets (128 rows of under 2^24 bytes), and enough tokens. us per launch
- * pair with the records at the 235B / 30B shapes, MFMA / row kernels: Q4_0 58 / 43 and 35 / 21 at
- * 4 tokens, about 59 / 72 and 35 / 33 at 6, 63 / 134 at 16; Q6_K 108 / 85 and 59 / 36 at 4, 112 /
- * 137 and 60 / 49 at 6, 64 / 109 (30B) at 16, where the row kernels take another pass. */
+ * offsets (128 rows of under 2^24 bytes), and enough tokens. From 9 tokens always: the row kernels
+ * then take another pass, also at the smallest (us at 9 tokens, row / MFMA kernels, records included:
+ * Q4_0 512x1024 12.0 / 9.6, 4096x4096 29.5 / 21.1; Q6_K 512x2048 29.4 / 22.1). At 5-8 tokens by rows:
+ * up to 4096 the row kernels' 16-row blocks fit the CUs once and win (5 tokens: Q4_0 4096x4096 18.6 /
+ * 20.9, 4096x8192 32.4 / 36.1; Q6_K 28.0 / 38.4, 51 / 72), above it not (Q4_0 6144x4096 23.7 / 21.1,
+ * 8192x2048 14.2 / 13.7; Q6_K 6144x4096 53 / 39, 10240x2048 30.4 / 23.9), save small matrices, where
+ * the records cost what is gained (Q4_0 6144x1024 8.5 / 9.3; Q6_K 8192x2048 20.2 / 22.8). */
 inline bool dense_mx_takes(const DenseArgs &a, int type)
 {
     if ((type != 2 && type != 3 && type != 14) || a.C % 256 || (type == 14 && a.rb % 4) || a.rb >= 1u << 24 || a.T > 4 * 65535)
@@ -149,7 +152,7 @@ inline bool dense_mx_takes(const DenseArgs &a, int type)
         if (a.m[i].rows < 128) return false;
         rows += a.m[i].rows;
     }
-    return a.T > 8 || (a.T > 4 && rows * a.C >= 1l << 24);
+    return a.T > 8 || (a.T > 4 && rows > 4096 && rows * a.C >= (type == 14 ? 5l << 22 : 1l << 24));
 }
 
 /* Widths of the chunked row kernels (others: the direct-read kernel), and whether those read pair

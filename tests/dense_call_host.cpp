@@ -195,6 +195,19 @@ static void capture_pairs()
     capturing = false;
 }
 
+/* at 5-8 tokens matrices that the row kernels' blocks cover in one pass over the CUs stay with them */
+static void few_rows()
+{
+    const struct { int type; int64_t rows, C; bool mfma; } m[] = {
+        { QMSG_T_Q6_K, 4096, 4096, false }, { QMSG_T_Q6_K, 4096, 8192, false }, { QMSG_T_Q6_K, 8192, 2048, false },
+        { QMSG_T_Q4_0, 4096, 8192, false }, { QMSG_T_Q4_0, 6144, 1024, false }, { QMSG_T_Q4_0, 8192, 2048, true },
+        { QMSG_T_Q6_K, 9216, 4096, true },  { QMSG_T_Q6_K, 151936, 2048, true },
+    };
+    for (const auto &k : m)
+        for (int T = 5; T <= 8; T++) CHECK(call(mat(k.type, k.rows, k.C), T) == QMSG_OK && launches.back().records == k.mfma);
+    CHECK(call(mat(QMSG_T_Q6_K, 128, 512), 9) == QMSG_OK && launches.back().records);
+}
+
 /* rows so long that a block's byte offsets (32 bits, the top one a flag) would not hold them stay off
  * the MFMA kernels */
 static void wide_rows()
@@ -232,6 +245,7 @@ int main(int argc, char **argv)
     else if (s == "no_memory") no_memory();
     else if (s == "no_buffer") no_buffer();
     else if (s == "capture_pairs") capture_pairs();
+    else if (s == "few_rows") few_rows();
     else if (s == "wide_rows") wide_rows();
     else if (s == "chain_lds") chain_lds();
     else return 2;
