@@ -35,6 +35,7 @@ namespace {
 
 constexpr int kChRows = 64;               /* rows of a block                                    */
 constexpr int kChResFloats = 16 * 1024;   /* inputs of up to 64 KiB are staged whole            */
+constexpr size_t kChResLds = 80 * 1024;   /* expert rows: where two blocks still share a CU     */
 
 /* A wave's staged chunk: NB blocks of 16 rows, BYTES per row, moved as 16-byte units to LDS rows
  * RS bytes apart (RS / 4 mod 64 a multiple of 4 that 16 rows spread over the banks). */
@@ -569,15 +570,19 @@ hipError_t launch_chain_rows(const char *name, const ChainRows &m, const ChainRo
     a.y_stride = m.y_stride;
     a.gu = gu;
     a.S = S;
-    /* an expert's slots are distinct tokens: up to 16 tokens every slot tile fits one
-     * instruction's columns, and its input rows LDS where T of them do */
-    const bool res = (size_t)T * m.cols <= kChResFloats && T <= 16;
     const dim3 grid = chain_grid((m.rows + (up ? 31 : 63)) / (up ? 32 : 64), max_tiles), block(256);
     const bool ok = with_type(m.type, [&](auto ty) {
         constexpr int TY = decltype(ty)::value;
         /* LDS of the inputs whole, or of stages; gate/up's results take less than either */
         static_assert(64 * 33 * 4 <= 4 * ChFmt<TY>::WAVE, "results of 32 slots fit in the row buffers");
         const size_t whole = ch_lds_res<TY>(T, m.cols);
+        /* an expert's slots are distinct tokens: up to 16 tokens every slot tile fits one
+         * instruction's columns, and its input rows LDS where T of them do. Grids of experts are
+         * several times the CUs, and a block that takes more than half a CU's LDS loses more than
+         * whole inputs gain (us a layer, whole / in stages: 30B, Q4_0 with Q8_0 down, 16 tokens
+         * 209 / 190; Q8_0 6 tokens 141 / 132; 235B --exact, Q4_0, 4 tokens 327 / 293; below the line
+         * 126 / 137 at one token) */
+        const bool res = T <= 16 && (size_t)T * m.cols <= kChResFloats && whole <= kChResLds;
         if (up) {
             if (res) QLAUNCH(name, (chain_rows_kernel<TY, 1, true, true>), grid, block, whole, st, a);
             else if (T <= 16) QLAUNCH(name, (chain_rows_kernel<TY, 1, true, false>), grid, block, ch_lds<TY>(1), st, a);

@@ -82,3 +82,17 @@ def test_chain_layer_many_tiles():
         parts = np.concatenate([ctx.moe(0, x[i:i + 11000]) for i in range(0, T, 11000)])
     assert np.array_equal(bits(out), bits(parts))
     assert np.array_equal(bits(out[-8:]), bits(L.moe(x[-8:])))
+
+
+@pytest.mark.parametrize("T", [11, 12])
+def test_chain_layer_staging(q, T):
+    """Gate/up inputs of 1024 floats on both sides of the LDS that two blocks share."""
+    E, X, K, F = 1024, 4, 2, 96
+    print(f"[case] chain layer staging T={T}", flush=True)
+    types = (orc.T_Q8_0,) * 3
+    L = et.typed_layer(E, X, K, F, types, 66)
+    x = orc.make_input(E, T, 67)
+    with q.Context(E, X, K, F, max_tokens=T) as ctx:
+        ctx.upload(0, L.router, *zip(types, (L.gate, L.up, L.down)))
+        out = ctx.moe(0, x)
+    assert np.array_equal(bits(out), bits(L.moe(x)))
