@@ -2984,32 +2984,6 @@ __device__ __forceinline__ void mx_wait_barrier()
     asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-#ifndef QMSG_MX_WIDE16_SLOTS
-#define QMSG_MX_WIDE16_SLOTS 8
-#endif
-#ifndef QMSG_MX_NARROW_GU
-#define QMSG_MX_NARROW_GU 8
-#endif
-#ifndef QMSG_MX_MID_NB
-#define QMSG_MX_MID_NB 2
-#endif
-#ifndef QMSG_MX_MID_NB_Q6
-#define QMSG_MX_MID_NB_Q6 1
-#endif
-/* staging of the 16-slot blocks: the weights in two buffers, the records in one
- * (mx_lds_bytes nb 3) */
-#ifndef QMSG_MX_WIDE16_NB_GU
-#define QMSG_MX_WIDE16_NB_GU 3
-#endif
-#ifndef QMSG_MX_WIDE16_NB_DN
-#define QMSG_MX_WIDE16_NB_DN 3
-#endif
-#ifndef QMSG_MX_WIDE16_NT
-#define QMSG_MX_WIDE16_NT 2
-#endif
-#ifndef QMSG_MX_WIDE16_NW
-#define QMSG_MX_WIDE16_NW 8
-#endif
 /* Waves per SIMD the MFMA kernel is built for: six where three double-buffered blocks' LDS
  * fits a CU, else four (the register budget follows: 80 or 128 VGPRs). */
 template <int TYPE, int WSG, int PPW, int NW, int NB, int NT>
@@ -3423,37 +3397,43 @@ static_assert(2 * mx_lds_bytes(14, 2) <= 160 * 1024, "two Q6_K blocks per CU");
  * 178 at r = 1.5, 187 / 199 at 2, 236 / 237 at 3, 287 / 269 at 4; mid / 8-slot blocks of 8 waves
  * 317-325 / 364-378 at 6; mid / wide 407-416 / 460-467 at 8, 571-620 / 581-593 at 12 (run to run),
  * 765-786 / 723-751 at 16. */
-constexpr int kMxWideSlotsGateUp = 12;
+/* Gate/up on narrow, mid, wide or wide16 blocks; down on thin blocks or those of 16 slots (Q4_0 / Q4_1
+ * wide16, Q6_K one tile per wave). */
 enum MxShape { kMxNarrow, kMxMid, kMxWide, kMxWide16, kMxThin };
 
-static MxShape mx_shape(const Shape &s, int T, int gu, int type)
+static MxShape mx_gateup_shape(const Shape &s, int T, int type)
 {
     const long NS = (long)T * s.K, act = s.X < NS ? s.X : NS;
-    if (!gu && NS < (type == 14 ? 6 : QMSG_MX_WIDE16_SLOTS) * act) return kMxThin;
-    if (type != 14 && QMSG_MX_WIDE16_SLOTS > 0 && NS >= QMSG_MX_WIDE16_SLOTS * act) return kMxWide16;
-    if (NS >= kMxWideSlotsGateUp * act) return kMxWide;
-    const long narrow_quarters = type == 14 ? 12 : QMSG_MX_NARROW_GU;
-    return 4 * NS < narrow_quarters * act ? kMxNarrow : kMxMid;
+    if (type != 14 && NS >= 8 * act) return kMxWide16;
+    if (type == 14 && NS >= 12 * act) return kMxWide;
+    return NS < (type == 14 ? 3 : 2) * act ? kMxNarrow : kMxMid;
 }
 
-template <int TYPE, int GU, int WSG, int PPW, int NW, int NB = 2, int NT = 2>
+static MxShape mx_down_shape(const Shape &s, int T, int type)
+{
+    const long NS = (long)T * s.K, act = s.X < NS ? s.X : NS;
+    return NS < (type == 14 ? 6 : 8) * act ? kMxThin : kMxWide16;
+}
+
+/* MODE: mx_kernel's (0 down, 1 gate/up, 2 dense, 3 down rows of alternating alignment). */
+template <int TYPE, int MODE, int WSG, int PPW, int NW, int NB = 2, int NT = 2>
 static void launch_mx_shape(const MxArgs &a, int rows, int maxt, hipStream_t st)
 {
     using Lay = MxLayout<TYPE, WSG, PPW, NW, NT>;
     const size_t lds = (size_t)mx_lds_bytes(TYPE, WSG, PPW, NW, NB, NT);
-    if constexpr (GU == 2) {
+    if constexpr (MODE == 2) {
         MxArgs b = a;
         int nblk = 0;
         for (int i = 0; i < b.d.nm; i++) {
             b.d.m[i].first_block = nblk;
             nblk += (b.d.m[i].rows + Lay::RWG - 1) / Lay::RWG;
         }
-        QLAUNCH("dense", (mx_kernel<TYPE, WSG, GU, PPW, NW, NB, NT>), dim3(nblk, (b.d.T + Lay::SWG - 1) / Lay::SWG),
+        QLAUNCH("dense", (mx_kernel<TYPE, WSG, MODE, PPW, NW, NB, NT>), dim3(nblk, (b.d.T + Lay::SWG - 1) / Lay::SWG),
                 dim3(64 * NW), lds, st, b);
         return;
     }
-    QLAUNCH(GU == 1 ? "gateup" : "down", (mx_kernel<TYPE, WSG, GU, PPW, NW, NB, NT>),
-            dim3(rows / (GU == 1 ? Lay::RWG / 2 : Lay::RWG), maxt, kTileN / Lay::SWG), dim3(64 * NW), lds, st, a);
+    QLAUNCH(MODE == 1 ? "gateup" : "down", (mx_kernel<TYPE, WSG, MODE, PPW, NW, NB, NT>),
+            dim3(rows / (MODE == 1 ? Lay::RWG / 2 : Lay::RWG), maxt, kTileN / Lay::SWG), dim3(64 * NW), lds, st, a);
 }
 
 /* Other shapes of the same kernel measured at the 512-token prefill: 32-slot blocks of 16
@@ -3462,28 +3442,27 @@ static void launch_mx_shape(const MxArgs &a, int rows, int maxt, hipStream_t st)
  * Staging buffers: the Q6_K gate/up blocks of 8 slots stage one chunk at a time (half the LDS, so
  * four blocks share a CU: the waves of other blocks cover each block's copy), the others two or,
  * 16-slot waves, two of weights and one of records. */
-template <int TYPE, int GU>
-static void launch_mx(const MxArgs &a, int rows, int maxt, MxShape shape, hipStream_t st)
+template <int TYPE>
+static void launch_mx_gateup(const MxArgs &a, int rows, int maxt, MxShape shape, hipStream_t st)
 {
-    if constexpr (!GU) {
-        if constexpr (TYPE == 14) {
-            if (a.rb % 4 && shape == kMxThin) return launch_mx_shape<14, 3, 1, 4, 4, 2, 1>(a, rows, maxt, st);
-            if (a.rb % 4) return launch_mx_shape<14, 3, 1, 8, 4, 3, 1>(a, rows, maxt, st);
+    if (shape == kMxNarrow) launch_mx_shape<TYPE, 1, 1, 2, 4>(a, rows, maxt, st);
+    else if (shape == kMxMid) launch_mx_shape<TYPE, 1, 1, 4, 4, TYPE == 14 ? 1 : 2>(a, rows, maxt, st);
+    else if constexpr (TYPE == 14) launch_mx_shape<14, 1, 2, 4, 8>(a, rows, maxt, st);
+    else launch_mx_shape<TYPE, 1, 1, 8, 4, 3>(a, rows, maxt, st);
+}
+
+template <int TYPE>
+static void launch_mx_down(const MxArgs &a, int rows, int maxt, MxShape shape, hipStream_t st)
+{
+    if constexpr (TYPE == 14) {
+        if (a.rb % 4) {
+            if (shape == kMxThin) launch_mx_shape<14, 3, 1, 4, 4, 2, 1>(a, rows, maxt, st);
+            else launch_mx_shape<14, 3, 1, 8, 4, 3, 1>(a, rows, maxt, st);
+            return;
         }
-        if (shape == kMxThin) return launch_mx_shape<TYPE, 0, 1, 4, 4, 2, 1>(a, rows, maxt, st);
-        if constexpr (TYPE == 14) return launch_mx_shape<14, 0, 1, 8, 4, 3, 1>(a, rows, maxt, st);
     }
-    if (shape == kMxWide) launch_mx_shape<TYPE, GU, 2, 4, 8>(a, rows, maxt, st);
-    else if (shape == kMxWide16) {
-        /* Q4_0 / Q4_1 only (mx_shape) */
-        if constexpr (TYPE != 14 && QMSG_MX_WIDE16_NT == 1)
-            launch_mx_shape<TYPE, GU, 1, 8, QMSG_MX_WIDE16_NW, GU ? QMSG_MX_WIDE16_NB_GU : QMSG_MX_WIDE16_NB_DN, 1>(
-                a, rows, maxt, st);
-        else if constexpr (TYPE != 14)
-            launch_mx_shape<TYPE, GU, 1, 8, 4, GU ? QMSG_MX_WIDE16_NB_GU : QMSG_MX_WIDE16_NB_DN>(a, rows, maxt, st);
-    }
-    else if (shape == kMxNarrow) launch_mx_shape<TYPE, GU, 1, 2, 4, 2>(a, rows, maxt, st);
-    else launch_mx_shape<TYPE, GU, 1, 4, 4, TYPE == 14 ? QMSG_MX_MID_NB_Q6 : QMSG_MX_MID_NB>(a, rows, maxt, st);
+    if (shape == kMxThin) launch_mx_shape<TYPE, 0, 1, 4, 4, 2, 1>(a, rows, maxt, st);
+    else launch_mx_shape<TYPE, 0, 1, 8, 4, 3, TYPE == 14 ? 1 : 2>(a, rows, maxt, st);
 }
 
 /* Whether the MFMA kernels take this layer: gate and up of one type (Q4_0, Q4_1, or Q6_K with
@@ -3519,9 +3498,9 @@ hipError_t launch_experts_mx(const Shape &s, const LayerDev &L, const Scratch &S
     a.rec = S.mxx;
     a.rec_out = S.mxa;
     a.S = S;
-    if (L.gate_type == 14) launch_mx<14, 1>(a, s.F, maxt, mx_shape(s, T, 1, 14), st);
-    else if (L.gate_type == 3) launch_mx<3, 1>(a, s.F, maxt, mx_shape(s, T, 1, 3), st);
-    else launch_mx<2, 1>(a, s.F, maxt, mx_shape(s, T, 1, 2), st);
+    if (L.gate_type == 14) launch_mx_gateup<14>(a, s.F, maxt, mx_gateup_shape(s, T, 14), st);
+    else if (L.gate_type == 3) launch_mx_gateup<3>(a, s.F, maxt, mx_gateup_shape(s, T, 3), st);
+    else launch_mx_gateup<2>(a, s.F, maxt, mx_gateup_shape(s, T, 2), st);
     if (!down_mx) {
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -3533,9 +3512,9 @@ hipError_t launch_experts_mx(const Shape &s, const LayerDev &L, const Scratch &S
     a.eb = L.down_eb;
     a.rec = S.mxa;
     a.rec_out = nullptr;
-    if (L.down_type == 14) launch_mx<14, 0>(a, s.E, maxt, mx_shape(s, T, 0, 14), st);
-    else if (L.down_type == 3) launch_mx<3, 0>(a, s.E, maxt, mx_shape(s, T, 0, 3), st);
-    else launch_mx<2, 0>(a, s.E, maxt, mx_shape(s, T, 0, 2), st);
+    if (L.down_type == 14) launch_mx_down<14>(a, s.E, maxt, mx_down_shape(s, T, 14), st);
+    else if (L.down_type == 3) launch_mx_down<3>(a, s.E, maxt, mx_down_shape(s, T, 3), st);
+    else launch_mx_down<2>(a, s.E, maxt, mx_down_shape(s, T, 2), st);
     const int n = T * s.E;
     QLAUNCH("combine", combine_kernel, dim3(n / (4 * combine_threads(s.E))), dim3(combine_threads(s.E)), 0, st, S, s.E, s.K, T, out);
     return hipGetLastError();
@@ -3562,9 +3541,9 @@ hipError_t launch_down_mx(const Shape &s, const LayerDev &L, const Scratch &S, f
     a.rec = S.mxa;
     a.rec_out = nullptr;
     a.S = S;
-    if (L.down_type == 14) launch_mx<14, 0>(a, s.E, maxt, mx_shape(s, T, 0, 14), st);
-    else if (L.down_type == 3) launch_mx<3, 0>(a, s.E, maxt, mx_shape(s, T, 0, 3), st);
-    else launch_mx<2, 0>(a, s.E, maxt, mx_shape(s, T, 0, 2), st);
+    if (L.down_type == 14) launch_mx_down<14>(a, s.E, maxt, mx_down_shape(s, T, 14), st);
+    else if (L.down_type == 3) launch_mx_down<3>(a, s.E, maxt, mx_down_shape(s, T, 3), st);
+    else launch_mx_down<2>(a, s.E, maxt, mx_down_shape(s, T, 2), st);
     const int n = T * s.E;
     QLAUNCH("combine", combine_kernel, dim3(n / (4 * combine_threads(s.E))), dim3(combine_threads(s.E)), 0, st, S, s.E, s.K, T, out);
     return hipGetLastError();
