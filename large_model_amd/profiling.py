@@ -20,28 +20,34 @@ import argparse
 import csv
 import glob
 import os
+import re
 import statistics
 import sys
 
-SHORT = (
-    ("route_small_kernel", "route"), ("route_big_kernel", "route"), ("select_kernel", "select"),
-    ("dispatch_kernel", "dispatch"), ("gateup_kernel", "gateup"), ("down_exact_kernel", "down"),
-    ("down_t1_kernel", "down"), ("down_small_kernel", "down"), ("act_quant_kernel", "actq"), ("swiglu_kernel", "swiglu"),
-    ("route_exact_kernel", "route"), ("exact_rows_kernel", "rows_f32"),
-    ("combine_kernel", "combine"), ("copy_kernel", "copy"), ("dense_kernel", "dense"),
-    ("dense_oct_kernel", "dense"), ("dense_tok_kernel", "dense"), ("dense_quant_kernel", "dquant"),
-    ("gateup_mfma_kernel", "gateup"), ("down_mfma_kernel", "down"), ("rmsnorm_kernel", "rmsnorm"),
-    ("add_rows_kernel", "add"),
-)
+# the launch names of the library's timing hook, by kernel
+SHORT = {
+    "route_small_kernel": "route", "route_big_kernel": "route", "route_norm_kernel": "route", "route_exact_kernel": "route",
+    "select_kernel": "select", "dispatch_wide_kernel": "dispatch", "gateup_kernel": "gateup", "down_t1_kernel": "down",
+    "down_small_kernel": "down", "act_quant_kernel": "actq", "swiglu_kernel": "swiglu", "combine_kernel": "combine",
+    "combine_any_kernel": "combine", "mx_input_kernel": "mxin", "quant_rows_kernel": "debug", "call_reset_kernel": "fill",
+    "copy_kernel": "copy", "dense_kernel": "dense", "dense_oct_kernel": "dense", "dense_tok_kernel": "dense",
+    "dense_any_kernel": "dense", "chain_dense_kernel": "dense", "dense_quant_kernel": "dquant",
+    "dense_mx_quant_kernel": "dquant", "rmsnorm_kernel": "rmsnorm", "add_rows_kernel": "add",
+}
 
 
 def short_name(kernel: str) -> str:
-    if "tile_rows_kernel" in kernel:       # last template argument: 1 = gate/up rows, 0 = down rows
-        return "gateup" if kernel.replace(" ", "").split(">")[0].endswith(",1") else "down"
-    for key, name in SHORT:
-        if key in kernel:
-            return name
-    return kernel.split("(")[0][:48]
+    m = re.search(r"(\w+_kernel)(?:<([^>]*)>)?", kernel)
+    if m is None:
+        return kernel.split("(")[0][:48]
+    name, args = m[1], (m[2] or "").replace(" ", "").split(",")
+    if name == "tile_rows_kernel":         # last template argument: 1 = gate/up rows, 0 = down rows
+        return "gateup" if args[-1] == "1" else "down"
+    if name == "mx_kernel":                # third: 1 = gate/up, 2 = dense rows, 0 and 3 = down
+        return {"1": "gateup", "2": "dense"}.get(args[2], "down")
+    if name == "chain_rows_kernel":        # third: gate and up at once, else the rows of one matrix
+        return "gateup" if args[2] == "true" else "rows_f32"
+    return SHORT.get(name, kernel.split("(")[0][:48])
 
 
 def _find(d: str, suffix: str) -> str:
