@@ -1083,8 +1083,8 @@ int qmsg_moe(qmsg_ctx *c, int layer, const float *xn, const float *h, int T, flo
     HIP_TRY(c, hipSetDevice(c->device));
     /* Small calls: the input through pinned memory and a copy kernel, and the layer's last launch
      * stores its rows to pinned memory. Pageable copies cost a runtime blit and a host round
-     * trip each. us per call, pinned / pageable: 30B 40 / 56 at one token, 85 / 126 at 8, 147 / 186
-     * at 32 (256 KiB in); 235B 50 / 59, 171 / 213, 255 / 298 at 16 (256 KiB). */
+     * trip each. us per call over four layers in turn, pinned / pageable: 30B 36 / 46 at one token, 83 /
+     * 121 at 8, 139 / 176 at 32 (256 KiB in); 235B 47 / 57, 163 / 201, 244 / 284 at 16 (256 KiB). */
     if (bytes <= kHostStage && !c->pin && hipHostMalloc((void **)&c->pin, 2 * kHostStage, hipHostMallocDefault) != hipSuccess) {
         c->pin = nullptr;                     /* the pageable copies below */
         (void)hipGetLastError();

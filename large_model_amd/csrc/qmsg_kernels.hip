@@ -4824,8 +4824,9 @@ __global__ void copy_kernel(uint4 *dst, const uint4 *src, size_t n)
 
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st)
 {
-    const size_t n = bytes / 16;
-    QLAUNCH("copy", copy_kernel, dim3(4096), dim3(256), 0, st, (uint4 *)dst, (const uint4 *)src, n);
+    const size_t n = bytes / 16, blocks = (n + 255) / 256;
+    const dim3 grid((unsigned)(blocks < 1 ? 1 : (blocks < 4096 ? blocks : 4096)));
+    QLAUNCH("copy", copy_kernel, grid, dim3(256), 0, st, (uint4 *)dst, (const uint4 *)src, n);
     return hipGetLastError();
 }
 

@@ -25,3 +25,19 @@ def test_host_call_sizes():
                 assert np.array_equal(out.view(np.uint32), want.view(np.uint32)), (T, l)
                 with pytest.raises(qmsg.QmsgError):
                     ctx.moe(2, x[:1])
+
+
+def test_copy_launch_sizes():
+    """The copy launch's grid follows the bytes: none, one unit, a block and one more, past its 4096 blocks."""
+    from large_model_amd import qmsg
+    print("[case] copy launch sizes", flush=True)
+    n = 4096 * 256 * 16 + 4096
+    x = np.random.default_rng(6).integers(0, 256, n, dtype=np.uint8)
+    with qmsg.Context(256, 16, 4, 128) as ctx:
+        d_x, d_y = ctx.device_alloc(n), ctx.device_alloc(n)
+        ctx.h2d(d_x, x)
+        for b in (0, 16, 4096, 4112, n):
+            ctx.h2d(d_y, np.zeros(n, np.uint8))
+            ctx._check(qmsg.lib.qmsg_calibrate_copy(ctx._h, d_y, d_x, b))
+            y = ctx.d2h(d_y, (n,), np.uint8)
+            assert np.array_equal(y[:b], x[:b]) and not y[b:].any(), b
