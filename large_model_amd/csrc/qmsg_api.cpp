@@ -921,7 +921,7 @@ static int run_layer_s(qmsg_ctx *c, const Scratch &S0, int layer, const float *d
     /* rows too long for every exact down kernel's LDS (n_ff_exp 14336: 8 KB per Q4_0 row) take
      * the MFMA down kernel on any path that allows it */
     const bool dn_long = dn_ok && T >= 2 && c->path != QMSG_PATH_EXACT && !down_exact_fits(s, d, T);
-    const bool dn_mx = dn_ok && (dn_long || (many && (forced || (autop && mx_auto_down(T, s.K, d.down_type)))));
+    const bool dn_mx = dn_ok && (dn_long || (many && (forced || (autop && mx_auto_down(T, s.K, s.F, d.down_type)))));
     if (ni) LAUNCH(c, "route", launch_route_norm(s, d, S, *ni, c->stream));
     else LAUNCH(c, "route", launch_route(s, d, S, d_xn, T, c->stream));
     LAUNCH(c, "select", launch_select(s, S, T, q4 ? 1 : 0, c->stream));

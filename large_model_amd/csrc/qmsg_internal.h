@@ -46,27 +46,32 @@ constexpr int kTileN = 32;
 constexpr int kMxRec = 128;
 
 /* The default path takes the MFMA kernels for gate/up once a batch averages kMxAutoQuarters / 4
- * slots per active expert, and for down from kMxDownMinSlotsQ4 slots (Q4_0 / Q4_1 rows) or
- * kMxDownMinSlotsQ6 (Q6_K rows). Measured per layer at the 235B shape, MFMA against the row
- * kernels (us; Q4 MFMA kernels on the 16x16x16 instructions): gate/up with the records each
- * needs 132.2 / 130.1 at 16 tokens, 114.2 / 107.1 at 12, and from 20 tokens (1.25 slots per
- * expert) 149.6 / 154.8; Q4_0 down after row-kernel gate/up, with the activation records it
- * needs: 41.3 / 41.5 at 6 tokens, 49.6 / 51.6 at 8, 55.8 / 62.1 at 12; Q6_K 41.6 / 32.9 at 2,
- * 49.4 / 46.2 at 3, 58.2 / 58.2 at 4, 105 / 118 at 8. */
+ * slots per active expert, and for down from kMxDownMinSlotsQ4 slots (Q4_0 / Q4_1 rows, and Q6_K rows
+ * of an odd number of super-blocks below kMxDownOddCols columns) or kMxDownMinSlotsQ6 (other Q6_K
+ * rows). Gate/up at the 235B shape, MFMA against the row kernels with the records each needs (us):
+ * 132.2 / 130.1 at 16 tokens, 114.2 / 107.1 at 12, and from 20 tokens (1.25 slots per expert) 149.6 /
+ * 154.8. Down after row-kernel gate/up, us of the layer, MFMA / row kernels: 235B Q4_0 89 / 86 at 4
+ * tokens, 118 / 119 at 6, 141 / 144 at 8, 217 / 228 at 16, 30B 56.2 / 53.7 at 6, 62.5 / 61.1 at 8, 71.3
+ * / 72.3 at 10 (Q4_1 the same within 2); 235B Q6_K 72 / 69 at 2, 93 / 95 at 3, 111 / 113 at 4, 129 / 153
+ * at 5. Odd rows: 1280 columns under 4096 rows 67 / 70 at 2, 101 / 118 at 4; 768 under 2048 (30B)
+ * 55.3 / 55.5 at 4, 62.7 / 59.8 at 5, 67.8 / 66.9 at 7, 72.5 / 72.0 at 8, 82 / 85 at 10; 768 under 1024
+ * 42.2 / 40.3 at 4, 52.2 / 51.6 at 8. */
 constexpr int kMxAutoQuarters = 5;
 /* Q6_K gate/up (its MFMA kernel unpacks 6-bit codes): from 2.5 slots per expert (streaming /
  * MFMA us: 442 / 487 at 32 tokens, 618 / 435 at 48) */
 constexpr int kMxAutoQuartersQ6 = 10;
 constexpr int kMxDownMinSlotsQ4 = 64;
 constexpr int kMxDownMinSlotsQ6 = 32;
+constexpr int kMxDownOddCols = 1024;
 inline bool mx_auto(int T, int K, int X, int gate_type)
 {
     const long NS = (long)T * K, act = X < NS ? X : NS;
     return 4 * NS >= (long)(gate_type == 14 ? kMxAutoQuartersQ6 : kMxAutoQuarters) * act;
 }
-inline bool mx_auto_down(int T, int K, int down_type)
+inline bool mx_auto_down(int T, int K, int F, int down_type)
 {
-    return (long)T * K >= (down_type == 14 ? kMxDownMinSlotsQ6 : kMxDownMinSlotsQ4);
+    const bool late = down_type != 14 || (F % 512 != 0 && F < kMxDownOddCols);
+    return (long)T * K >= (late ? kMxDownMinSlotsQ4 : kMxDownMinSlotsQ6);
 }
 
 /* One-token batches (n_used <= 8) are routed inside the gate/up kernel instead of by a

@@ -208,6 +208,14 @@ static void few_rows()
     CHECK(call(mat(QMSG_T_Q6_K, 128, 512), 9) == QMSG_OK && launches.back().records);
 }
 
+/* down rows of an odd number of Q6_K super-blocks: short ones take the MFMA kernels from 64 slots */
+static void odd_down()
+{
+    CHECK(!qmsg::mx_auto_down(5, 8, 768, 14) && !qmsg::mx_auto_down(7, 8, 256, 14) && qmsg::mx_auto_down(8, 8, 768, 14));
+    CHECK(qmsg::mx_auto_down(4, 8, 1280, 14) && qmsg::mx_auto_down(4, 8, 1536, 14) && qmsg::mx_auto_down(4, 8, 512, 14));
+    CHECK(!qmsg::mx_auto_down(3, 8, 1280, 14) && !qmsg::mx_auto_down(7, 8, 768, 2) && qmsg::mx_auto_down(8, 8, 768, 2));
+}
+
 /* rows so long that a block's byte offsets (32 bits, the top one a flag) would not hold them stay off
  * the MFMA kernels */
 static void wide_rows()
@@ -246,6 +254,7 @@ int main(int argc, char **argv)
     else if (s == "no_buffer") no_buffer();
     else if (s == "capture_pairs") capture_pairs();
     else if (s == "few_rows") few_rows();
+    else if (s == "odd_down") odd_down();
     else if (s == "wide_rows") wide_rows();
     else if (s == "chain_lds") chain_lds();
     else return 2;

@@ -31,7 +31,7 @@ def test_record_buffer(exe, scenario):
     run(exe, scenario)
 
 
-@pytest.mark.parametrize("scenario", ["chain_lds", "wide_rows"])
+@pytest.mark.parametrize("scenario", ["chain_lds", "wide_rows", "odd_down"])
 def test_kernel_limits(exe, scenario):
     run(exe, scenario)
 
