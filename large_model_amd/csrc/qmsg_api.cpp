@@ -658,7 +658,8 @@ static int dense_check(qmsg_ctx *c, int type, int64_t rows, int64_t cols, const 
     if (direct && !exact_only && type != QMSG_T_F32 && cols / 32 * 48 > 160 * 1024)
         return fail(c, QMSG_E_UNSUPPORTED, "%s: cols %lld is not a multiple of %d and above %d", what, (long long)cols,
                     type == QMSG_T_Q6_K ? 2048 : 256, 160 * 1024 / 48 * 32);
-    /* the fp32-chain kernel stages one input row of cols floats in LDS */
+    /* the widths fp32-chain rows are taken at (one input row in 160 KiB); the kernels, which stage wider
+     * inputs in pieces, would run any */
     if (exact_only && cols * 4 > 160 * 1024)
         return fail(c, QMSG_E_UNSUPPORTED, "%s: F16 / Q8_0 rows above %d columns", what, 160 * 1024 / 4);
     return QMSG_OK;
@@ -780,7 +781,7 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
         const int t = c->mats[(size_t)ids[i]].type;
         exact = exact || t == QMSG_T_F16 || t == QMSG_T_Q8_0;
     }
-    if (exact && C * 4 > 160 * 1024)
+    if (exact && C * 4 > 160 * 1024)                /* as dense_check */
         return fail(c, QMSG_E_UNSUPPORTED, "qmsg_matmul_n: fp32-chain rows above %d columns", 160 * 1024 / 4);
     /* launches of up to kDenseMats matrices of one type, in argument order */
     struct Group {

@@ -4665,7 +4665,8 @@ hipError_t launch_layer_slots(const Shape &s, const LayerDev &L, const Scratch &
         /* gate and up of one type in one launch */
         const bool pair = i == 0 && m[1].type == m[0].type;
         if (chain_rows(m[i].type)) {
-            /* the widths this path takes: four input rows (or the batch's) in 160 KiB */
+            /* the widths this path is open to: four input rows (or the batch's) in 160 KiB. The chain
+             * kernels have no such limit; wider calls have always been refused */
             if ((size_t)min(4, T) * m[i].cols * 4 > 160 * 1024) return hipErrorInvalidValue;
             ChainRows r = m[i];
             if (pair) {
