@@ -55,6 +55,34 @@ def test_chain_non_finite(q, bad):
     assert np.array_equal(bits(y)[fine], bits(want)[fine])
 
 
+@pytest.mark.parametrize("T", [3, 18])
+@pytest.mark.parametrize("type_", [orc.T_F32, orc.T_F16, orc.T_Q8_0])
+def test_chain_subnormal_results(q, type_, T):
+    """Chains whose products and sums are subnormal, pass through zero, or move between subnormal and
+    normal step by step."""
+    cols, rows = 288, 70
+    print(f"[case] chain subnormal type {type_} T={T}", flush=True)
+    rng = np.random.default_rng(52 + T)
+    x = orc.make_input(cols, T, 53)
+    if type_ == orc.T_F32:
+        w = np.ldexp(rng.standard_normal((rows, cols)), rng.integers(-80, -50, (rows, cols))).astype(np.float32)
+        w = np.ascontiguousarray(w).view(np.uint8).ravel()
+        x *= np.ldexp(np.float32(1), rng.integers(-104, -75, x.shape)).astype(np.float32)
+    else:
+        w = et.expert_bytes(type_, rows, cols, 1, 54)                 # values or scales down to 2^-24
+        if type_ == orc.T_F16:
+            w = (w.view(np.float16) * np.float16(1e-3)).view(np.uint8)
+        x *= np.ldexp(np.float32(1), rng.integers(-136, -113 if type_ == orc.T_F16 else -125, x.shape)).astype(np.float32)
+    x[1] = -x[0]
+    want = orc.matmul_n([(type_, w, rows, cols)], x, exact=True)[0]
+    small = np.abs(want) < np.finfo(np.float32).tiny
+    assert (small & (want != 0)).mean() > 0.3                         # most results are themselves subnormal
+    with q.Context(256, 16, 4, 128, max_tokens=1) as ctx:
+        ctx.set_path(q.PATH_FP32)
+        y = ctx.matmul_n([ctx.mat_upload(type_, w, rows, cols)], x)[0]
+    assert np.array_equal(bits(y), bits(want))
+
+
 @pytest.mark.parametrize("T", [1, 5, 16, 17, 40, 70])
 @pytest.mark.parametrize("types", [(orc.T_Q8_0,) * 3, (orc.T_F16,) * 3, (orc.T_Q8_0, orc.T_F16, orc.T_Q8_0)])
 def test_chain_layer(q, T, types):
