@@ -36,10 +36,16 @@ SHORT = {
 }
 
 
+def full_name(kernel: str) -> str:
+    """A kernel's name and template arguments, without its parameters."""
+    return kernel.replace("(anonymous namespace)::", "").split("(")[0]
+
+
 def short_name(kernel: str) -> str:
+    kernel = full_name(kernel)
     m = re.search(r"(\w+_kernel)(?:<([^>]*)>)?", kernel)
     if m is None:
-        return kernel.split("(")[0][:48]
+        return kernel[:48]
     name, args = m[1], (m[2] or "").replace(" ", "").split(",")
     if name == "tile_rows_kernel":         # last template argument: 1 = gate/up rows, 0 = down rows
         return "gateup" if args[-1] == "1" else "down"
@@ -47,7 +53,7 @@ def short_name(kernel: str) -> str:
         return {"1": "gateup", "2": "dense"}.get(args[2], "down")
     if name == "chain_rows_kernel":        # third: gate and up at once, else the rows of one matrix
         return "gateup" if args[2] == "true" else "rows_f32"
-    return SHORT.get(name, kernel.split("(")[0][:48])
+    return SHORT.get(name, kernel[:48])
 
 
 def _find(d: str, suffix: str) -> str:
@@ -64,7 +70,7 @@ def stats(d: str) -> list[str]:
         name = r["Name"]
         out.append(f"{short_name(name):10s} {int(r['Calls']):9d} {float(r['AverageNs']) / 1e3:9.3f} "
                    f"{float(r['MinNs']) / 1e3:9.3f} {float(r['MaxNs']) / 1e3:9.3f} {float(r['Percentage']):6.2f}%  "
-                   f"{name[:90]}")
+                   f"{full_name(name)[:90]}")
     return out
 
 
@@ -97,7 +103,7 @@ def counters(dirs: list[str]) -> list[str]:
     out = []
     for k in sorted(per_kernel):
         cs = per_kernel[k]
-        out.append(f"{k.split('(')[0]}  [{max(len(v) for v in cs.values())} dispatches]")
+        out.append(f"{full_name(k)}  [{max(len(v) for v in cs.values())} dispatches]")
         for c in sorted(cs):
             out.append(f"   {c:32s} {sum(cs[c]) / len(cs[c]):18.0f}")
     return out

@@ -3,7 +3,7 @@ import glob
 import os
 import re
 
-from large_model_amd.profiling import short_name
+from large_model_amd.profiling import counters, short_name
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "large_model_amd", "csrc")
 
@@ -28,3 +28,13 @@ def test_short_names_by_template_argument():
                        ("void qmsg::(anonymous namespace)::chain_rows_kernel<8, 2, false, false>(qmsg::ChainArgs)", "rows_f32"),
                        ("__amd_rocclr_copyBuffer", "__amd_rocclr_copyBuffer")):
         assert short_name(full) == name, full
+
+
+def test_counters_keep_kernels_of_an_anonymous_namespace_apart(tmp_path):
+    rows = ["Dispatch_Id,Kernel_Name,Counter_Name,Counter_Value"]
+    for i, arg in enumerate(("true", "false", "true")):
+        rows.append(f'{i},"void qmsg::(anonymous namespace)::chain_rows_kernel<8, 2, {arg}, false>(qmsg::ChainArgs)",SQ_WAVES,{i + 1}')
+    (tmp_path / "p_counter_collection.csv").write_text("\n".join(rows) + "\n")
+    out = counters([str(tmp_path)])
+    assert out[0].startswith("void qmsg::chain_rows_kernel<8, 2, false, false>  [1 ") and out[1].split() == ["SQ_WAVES", "2"]
+    assert out[2].startswith("void qmsg::chain_rows_kernel<8, 2, true, false>  [2 ") and out[3].split() == ["SQ_WAVES", "2"]
