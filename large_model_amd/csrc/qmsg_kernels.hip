@@ -630,6 +630,13 @@ __global__ __launch_bounds__(256) void select_kernel(SelectArgs a, int do_dispat
     PHASE(0, 7);
 }
 
+/* The slots of a small batch sorted by one wave in a launch of its own (slot kernels). */
+__global__ __launch_bounds__(64) void dispatch_kernel(SelectArgs a)
+{
+    __shared__ int cnt[kMaxExperts], cur[kMaxExperts], tok[kMaxExperts];
+    dispatch_slots(a, a.S.sel, cnt, cur, tok);
+}
+
 /* Inclusive sum over the block's first kMaxExperts threads (4 waves); others return 0. */
 __device__ __forceinline__ int experts_scan(int v, int *wsum)
 {
@@ -742,6 +749,23 @@ hipError_t launch_select(const Shape &s, const Scratch &S, int T, int gateup_rou
      * 16-wave dispatch launch (measured 5 us less per layer at 48 and 64 tokens) */
     QLAUNCH("select", select_kernel, dim3(T), dim3(256), 0, st, a, T <= 16 ? 1 : 0);
     if (T > 16) QLAUNCH("dispatch", dispatch_wide_kernel, dim3(1), dim3(64 * kDispWaves), 0, st, a);
+    return hipGetLastError();
+}
+
+/* launch_select for the slot and fp32-chain kernels: up to 128 slots are sorted by one wave in a launch
+ * of its own, which small layers end sooner than with the ticketed last block (up to 16 tokens) or the
+ * 16-wave launch (us a layer: E 288, Q4_0, 4 tokens 27.7 / 28.6, 17 tokens 29.9 / 31.2, 24 tokens 36.1 /
+ * 37.9; 96 and 128 tokens, of 192 and 256 slots, 61.5 / 61.3 and 69.7 / 69.5). */
+static hipError_t launch_select_slots(const Shape &s, const Scratch &S, int T, hipStream_t st)
+{
+    if (T == 1 || T * s.K > 128) return launch_select(s, S, T, 0, st);
+    SelectArgs a;
+    a.X = s.X;
+    a.K = s.K;
+    a.T = T;
+    a.S = S;
+    QLAUNCH("select", select_kernel, dim3(T), dim3(256), 0, st, a, 0);
+    QLAUNCH("dispatch", dispatch_kernel, dim3(1), dim3(64), 0, st, a);
     return hipGetLastError();
 }
 
@@ -4642,7 +4666,7 @@ hipError_t launch_layer_slots(const Shape &s, const LayerDev &L, const Scratch &
         if (e != hipSuccess) return e;
     }
     if (!down_only) {
-        const hipError_t e = launch_select(s, S, T, 0, st);
+        const hipError_t e = launch_select_slots(s, S, T, st);
         if (e != hipSuccess) return e;
     }
     const int maxact = s.X < T * s.K ? s.X : T * s.K;

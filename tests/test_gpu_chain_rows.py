@@ -83,10 +83,11 @@ def test_chain_subnormal_results(q, type_, T):
     assert np.array_equal(bits(y), bits(want))
 
 
-@pytest.mark.parametrize("T", [1, 5, 16, 17, 40, 70])
+@pytest.mark.parametrize("T", [1, 5, 16, 17, 40, 64, 65, 70])
 @pytest.mark.parametrize("types", [(orc.T_Q8_0,) * 3, (orc.T_F16,) * 3, (orc.T_Q8_0, orc.T_F16, orc.T_Q8_0)])
 def test_chain_layer(q, T, types):
-    """Few experts, so that slot tiles hold 16, 17, 32 and a tail of slots."""
+    """Few experts, so that slot tiles hold 16, 17, 32 and a tail of slots; 128 and 130 slots are sorted by
+    one wave and by sixteen."""
     E, X, K, F = 288, 4, 2, 96
     print(f"[case] chain layer {types} T={T}", flush=True)
     L = et.typed_layer(E, X, K, F, types, 60)
