@@ -145,6 +145,7 @@ struct qmsg_ctx {
     /* grow-on-demand buffers of the dense products: input records, host-call staging */
     void *dense_xqk = nullptr;
     size_t dense_xqk_bytes = 0;
+    bool dense_xqk_held = false;            /* by a captured call: never freed before the context */
     void *dense_io = nullptr;
     size_t dense_io_bytes = 0;
     /* pinned rows of the host-buffer layer call (kHostStage bytes in, as many out), on first use */
@@ -816,14 +817,20 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
     }
     /* The record buffer, where a launch of this call reads it: the MFMA records, or the smaller pair
      * records of the row kernels, which take over without memory for the others (of fewer than
-     * kDenseQuantT rows they read none). A later, larger call replaces the buffer, so a graph must
+     * kDenseQuantT rows they read none). A later, larger call replaces the buffer, so a graph does
      * not hold it where it need not: captured calls of fewer than kDenseQuantT rows always take the
-     * row kernels, larger ones what the buffer already holds. */
+     * row kernels, larger ones what the buffer already holds. A buffer that a captured call was given
+     * is kept until the context is destroyed. */
     const size_t recs = dense_record_bytes((size_t)T, (size_t)C);
-    if (mfma && (T < kDenseQuantT || c->dense_xqk_bytes < recs)) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
-        if (cap != hipStreamCaptureStatusNone && c->dense_xqk_bytes >= pairs) mfma = false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (mfma || pairs) HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
+    const bool captured = cap != hipStreamCaptureStatusNone;
+    if (captured && (T < kDenseQuantT || c->dense_xqk_bytes < recs) && c->dense_xqk_bytes >= pairs) mfma = false;
+    if (c->dense_xqk_bytes < (mfma ? recs : pairs) && c->dense_xqk_held) {
+        c->scratch_allocs.push_back(c->dense_xqk);
+        c->dense_xqk = nullptr;
+        c->dense_xqk_bytes = 0;
+        c->dense_xqk_held = false;
     }
     int rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, mfma ? recs : pairs);
     if (rc == QMSG_E_NOMEM && mfma) {
@@ -831,6 +838,7 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
         rc = grow(c, &c->dense_xqk, &c->dense_xqk_bytes, pairs);
     }
     if (rc) return rc;
+    if (captured && (mfma || pairs)) c->dense_xqk_held = true;
     const uint64_t epoch = next_epoch();
     bool records = false;
     for (const Group &g : groups) {

@@ -138,6 +138,23 @@ static void capture_small()
     }
 }
 
+/* captured calls of 8 and more rows, on MFMA and on pair records, and larger calls after them */
+static void capture_large()
+{
+    const int big = mat(QMSG_T_Q4_0, 8192, 4096), few = mat(QMSG_T_Q4_0, 64, 4096);
+    std::vector<size_t> held;
+    for (int T : { 8, 16, 64 })
+        for (int id : { big, few }) {
+            CHECK(call(id, T) == QMSG_OK);
+            capturing = true;
+            held.push_back(launches.size());
+            CHECK(call(id, T) == QMSG_OK && launches.back().xqk);
+            capturing = false;
+            CHECK(call(big, 2 * T) == QMSG_OK);         /* replaces the buffer */
+            for (size_t n : held) CHECK(launches_safe(n, n + 1));
+        }
+}
+
 /* no memory for the record buffer: 5-7 rows fall to the row kernels, 8 and more to the smaller pair
  * records, and with none for those either the call says so; nothing of it reaches the next call */
 static void no_memory()
@@ -250,6 +267,7 @@ int main(int argc, char **argv)
     if (argc != 2 || qmsg_create(&ctx, 0, &cfg, 1, 1) != QMSG_OK) return 2;
     const std::string s = argv[1];
     if (s == "capture_small") capture_small();
+    else if (s == "capture_large") capture_large();
     else if (s == "no_memory") no_memory();
     else if (s == "no_buffer") no_buffer();
     else if (s == "capture_pairs") capture_pairs();
@@ -259,5 +277,9 @@ int main(int argc, char **argv)
     else if (s == "chain_lds") chain_lds();
     else return 2;
     qmsg_destroy(ctx);
+    if (!live.empty()) {
+        fprintf(stderr, "%zu allocations outlive the context\n", live.size());
+        return 1;
+    }
     return 0;
 }

@@ -26,7 +26,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("scenario", ["capture_small", "no_memory", "no_buffer", "capture_pairs", "few_rows"])
+@pytest.mark.parametrize("scenario", ["capture_small", "capture_large", "no_memory", "no_buffer", "capture_pairs", "few_rows"])
 def test_record_buffer(exe, scenario):
     run(exe, scenario)
 

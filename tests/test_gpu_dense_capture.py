@@ -21,7 +21,7 @@ def hip_lib():
     return hip
 
 
-@pytest.mark.parametrize("T", [5, 7])
+@pytest.mark.parametrize("T", [5, 7, 8, 16])
 def test_capture_survives_growth(T):
     from large_model_amd import qmsg
     hip, vp = hip_lib(), ctypes.c_void_p
@@ -44,7 +44,7 @@ def test_capture_survives_growth(T):
         assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
         assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
         try:
-            for n in (16, big, 2 * big, 4 * big):     # each larger call replaces the buffer
+            for n in (32, big, 2 * big, 4 * big):     # each larger call replaces the buffer
                 ctx.matmul_n_device([i], d_x, n, [d_yb])
                 ctx.h2d(d_y, np.zeros((T, rows), np.float32))
                 assert hip.hipGraphLaunch(exe, st) == 0
