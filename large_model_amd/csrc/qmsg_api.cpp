@@ -82,15 +82,15 @@ std::vector<ScratchItem> scratch_items(const qmsg_cfg &cfg, size_t T, Scratch *S
     };
 }
 
+/* Host-buffer layer calls of up to this many input bytes pass through pinned memory that the kernels
+ * read and write themselves (qmsg_moe). */
+constexpr size_t kHostStage = 256 * 1024;
+
 /* ---- the allocation-free layer call (qmsg_moe_device_noalloc) ----
  * Its scratch arrays live in this file-scope device array, one copy per GPU, held until the
  * process ends. Host code never passes `scratch` itself (in host code the name is only a
  * stand-in): each device's address comes from hipGetSymbolAddress, taken once per device
  * with that device current (in qmsg_create), and only that address is used. */
-/* Host-buffer layer calls of up to this many input bytes pass through pinned memory that the kernels
- * read and write themselves (qmsg_moe). */
-constexpr size_t kHostStage = 256 * 1024;
-
 constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;
 constexpr int kMaxDevices = 64;
 __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];

@@ -21,8 +21,11 @@
  * with the lane-swap instructions. Inputs sit in LDS as [row][block][g][8]: all of them before
  * the loop where they fit (RES), else a few blocks at a time with one barrier each.
  *
- * Bound: the matrix pipe at batch sizes (padding of partly filled 16-column tiles included), the
- * one chain's latency at one token. The 30B shape with Q8_0 experts, us, against one lane per row
+ * Bound: at one token the one chain's latency. At batch sizes no unit is full (30B, Q8_0, 201 tokens
+ * of a skewed load, gate/up / down): the matrix pipe is busy 0.49 / 0.44 of the time, partly filled
+ * 16-column tiles included, LDS 0.37 / 0.35, over half of that bank conflicts (inputs are stored as
+ * single words); two blocks per CU leave 1.7 waves per SIMD, which wait to issue for 0.64 / 0.60 of
+ * their cycles. The 30B shape with Q8_0 experts, us, against one lane per row
  * and four slots per pass on the vector ALU: gate/up with SwiGLU 19 (45 + 7), down 9.8 (20) at
  * one token; 254 and 135 (together 5744) at 201 tokens of a skewed load, the layer 383 (5860). */
 #include <type_traits>

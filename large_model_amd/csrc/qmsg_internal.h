@@ -136,8 +136,8 @@ struct DenseArgs {
     const uint8_t *xqk;     /* [T][C/64] pair records, or NULL: the kernel quantises x */
 };
 
-/* Batches of at least this many rows are quantised once by a separate launch; smaller ones
- * inside every dense block. */
+/* Dense row kernels: batches of at least this many rows are quantised once by a separate launch,
+ * smaller ones inside every block. */
 constexpr int kDenseQuantT = 8;
 /* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
  * read (Q6_K: 4-byte aligned), a block's rows in each matrix and their bytes in the 31 bits of its
