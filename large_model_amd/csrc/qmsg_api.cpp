@@ -818,14 +818,15 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
     /* The record buffer, where a launch of this call reads it: the MFMA records, or the smaller pair
      * records of the row kernels, which take over without memory for the others (of fewer than
      * kDenseQuantT rows they read none). A later, larger call replaces the buffer, so a graph does
-     * not hold it where it need not: captured calls of fewer than kDenseQuantT rows always take the
-     * row kernels, larger ones what the buffer already holds. A buffer that a captured call was given
+     * not hold it where it need not: captured calls of fewer than kDenseQuantT rows take the row
+     * kernels at every width these are sure to take, others what the buffer already holds. A buffer that a captured call was given
      * is kept until the context is destroyed. */
     const size_t recs = dense_record_bytes((size_t)T, (size_t)C);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (mfma || pairs) HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
     const bool captured = cap != hipStreamCaptureStatusNone;
-    if (captured && (T < kDenseQuantT || c->dense_xqk_bytes < recs) && c->dense_xqk_bytes >= pairs) mfma = false;
+    const bool row_first = T < kDenseQuantT && C <= kDenseRowCols;
+    if (captured && (row_first || c->dense_xqk_bytes < recs) && c->dense_xqk_bytes >= pairs) mfma = false;
     if (c->dense_xqk_bytes < (mfma ? recs : pairs) && c->dense_xqk_held) {
         c->scratch_allocs.push_back(c->dense_xqk);
         c->dense_xqk = nullptr;

@@ -139,6 +139,10 @@ struct DenseArgs {
 /* Dense row kernels: batches of at least this many rows are quantised once by a separate launch,
  * smaller ones inside every block. */
 constexpr int kDenseQuantT = 8;
+/* Rows of more columns can be too long for the row kernels' LDS at several tokens (Q6_K above 16,384,
+ * Q4_0 / Q4_1 above 25,600): there the MFMA kernels stay first. */
+constexpr int kDenseRowCols = 16384;
+
 /* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
  * read (Q6_K: 4-byte aligned), a block's rows in each matrix and their bytes in the 31 bits of its
  * offsets (128 rows of under 2^24 bytes), and enough tokens. From 9 tokens always: the row kernels
@@ -157,7 +161,9 @@ inline bool dense_mx_takes(const DenseArgs &a, int type)
         if (a.m[i].rows < 128) return false;
         rows += a.m[i].rows;
     }
-    return a.T > 8 || (a.T > 4 && rows > 4096 && rows * a.C >= (type == 14 ? 5l << 22 : 1l << 24));
+    if (a.T > 8) return true;
+    if (a.C > kDenseRowCols) return a.T > 4 && rows * a.C >= 1l << 24;
+    return a.T > 4 && rows > 4096 && rows * a.C >= (type == 14 ? 5l << 22 : 1l << 24);
 }
 
 /* Widths of the chunked row kernels (others: the direct-read kernel), and whether those read pair

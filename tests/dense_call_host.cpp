@@ -95,6 +95,7 @@ static int mat(int type, int64_t rows, int64_t cols)
 {
     static uint8_t data[16];
     const uint64_t rb = type == QMSG_T_Q4_0 ? (uint64_t)cols / 32 * 18
+                        : type == QMSG_T_Q4_1 ? (uint64_t)cols / 32 * 20
                         : type == QMSG_T_Q8_0 ? (uint64_t)cols / 32 * 34
                         : type == QMSG_T_Q6_K ? (uint64_t)cols / 256 * 210 : (uint64_t)cols * 4;
     const qmsg_mat m = { type, rows, cols, rb, data };
@@ -136,6 +137,14 @@ static void capture_small()
         CHECK(launches_safe(n, n + 1));
         CHECK(call(big, T) == QMSG_OK && launches.back().records);
     }
+    /* rows that only the MFMA kernels take: the buffer that is there, kept */
+    const int wide = mat(QMSG_T_Q4_0, 1024, 32768);
+    CHECK(call(wide, 6) == QMSG_OK && launches.back().records);
+    capturing = true;
+    const size_t n = launches.size();
+    CHECK(call(wide, 6) == QMSG_OK && launches[n].records);
+    capturing = false;
+    CHECK(call(wide, 64) == QMSG_OK && launches_safe(n, n + 1));
 }
 
 /* captured calls of 8 and more rows, on MFMA and on pair records, and larger calls after them */
@@ -219,6 +228,8 @@ static void few_rows()
         { QMSG_T_Q6_K, 4096, 4096, false }, { QMSG_T_Q6_K, 4096, 8192, false }, { QMSG_T_Q6_K, 8192, 2048, false },
         { QMSG_T_Q4_0, 4096, 8192, false }, { QMSG_T_Q4_0, 6144, 1024, false }, { QMSG_T_Q4_0, 8192, 2048, true },
         { QMSG_T_Q6_K, 9216, 4096, true },  { QMSG_T_Q6_K, 151936, 2048, true },
+        /* rows too long for the row kernels' LDS at several tokens */
+        { QMSG_T_Q4_0, 1024, 32768, true }, { QMSG_T_Q4_1, 256, 65536, true }, { QMSG_T_Q6_K, 704, 24576, true },
     };
     for (const auto &k : m)
         for (int T = 5; T <= 8; T++) CHECK(call(mat(k.type, k.rows, k.C), T) == QMSG_OK && launches.back().records == k.mfma);

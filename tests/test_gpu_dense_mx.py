@@ -42,7 +42,8 @@ def test_dense_mx_edges(q, T, cols):
 
 @pytest.mark.parametrize("type_,rows,cols,T", [(orc.T_Q4_0, 1024, 256, 1601), (orc.T_Q6_K, 1090, 512, 2050),
                                                (orc.T_Q4_0, 4160, 4096, 6), (orc.T_Q6_K, 8192, 2048, 5),
-                                               (orc.T_Q6_K, 10240, 2048, 5)])
+                                               (orc.T_Q6_K, 10240, 2048, 5), (orc.T_Q4_0, 256, 65536, 6),
+                                               (orc.T_Q6_K, 704, 24576, 7)])
 def test_dense_mx_large_grids(q, type_, rows, cols, T):
     """The block shapes of large grids, and few tokens on large matrices."""
     print(f"[case] dense mx large type {type_} {rows}x{cols} T={T}", flush=True)
