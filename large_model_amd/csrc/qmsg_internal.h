@@ -146,8 +146,9 @@ constexpr int kDenseRowCols = 16384;
 /* Whether a call's matrices take the MFMA kernels: rows in whole staged chunks that the LDS DMA can
  * read (Q6_K: 4-byte aligned), a block's rows in each matrix and their bytes in the 31 bits of its
  * offsets (128 rows of under 2^24 bytes), and enough tokens. From 9 tokens always: the row kernels
- * then take another pass, also at the smallest (us at 9 tokens, row / MFMA kernels, records included:
- * Q4_0 512x1024 12.0 / 9.6, 4096x4096 29.5 / 21.1; Q6_K 512x2048 29.4 / 22.1). At 5-8 tokens by rows:
+ * then take another pass, and the smallest lose nothing (us at 9 tokens, row / MFMA kernels, records
+ * included: Q4_0 128x256 6.9 / 6.9, 512x1024 12.0 / 9.6, 4096x4096 29.5 / 21.1; Q6_K 130x512 13.2 / 9.1,
+ * 512x2048 29.4 / 22.1). At 5-8 tokens by rows:
  * up to 4096 the row kernels' 16-row blocks fit the CUs once and win (5 tokens: Q4_0 4096x4096 18.6 /
  * 20.9, 4096x8192 32.4 / 36.1; Q6_K 28.0 / 38.4, 51 / 72), above it not (Q4_0 6144x4096 23.7 / 21.1,
  * 8192x2048 14.2 / 13.7; Q6_K 6144x4096 53 / 39, 10240x2048 30.4 / 23.9), save small matrices, where
