@@ -27,7 +27,7 @@ import sys
 # the launch names of the library's timing hook, by kernel
 SHORT = {
     "route_small_kernel": "route", "route_big_kernel": "route", "route_norm_kernel": "route", "route_exact_kernel": "route",
-    "select_kernel": "select", "dispatch_wide_kernel": "dispatch", "gateup_kernel": "gateup", "down_t1_kernel": "down",
+    "select_kernel": "select", "dispatch_kernel": "dispatch", "dispatch_wide_kernel": "dispatch", "gateup_kernel": "gateup", "down_t1_kernel": "down",
     "down_small_kernel": "down", "act_quant_kernel": "actq", "swiglu_kernel": "swiglu", "combine_kernel": "combine",
     "combine_any_kernel": "combine", "mx_input_kernel": "mxin", "quant_rows_kernel": "debug", "call_reset_kernel": "fill",
     "copy_kernel": "copy", "dense_kernel": "dense", "dense_oct_kernel": "dense", "dense_tok_kernel": "dense",
