@@ -819,8 +819,8 @@ int qmsg_matmul_n_device(qmsg_ctx *c, const int *ids, int nW, const float *d_x, 
      * records of the row kernels, which take over without memory for the others (of fewer than
      * kDenseQuantT rows they read none). A later, larger call replaces the buffer, so a graph does
      * not hold it where it need not: captured calls of fewer than kDenseQuantT rows take the row
-     * kernels at every width these are sure to take, others what the buffer already holds. A buffer that a captured call was given
-     * is kept until the context is destroyed. */
+     * kernels at every width these are sure to take, others what the buffer already holds. A buffer
+     * that a captured call was given is kept until the context is destroyed. */
     const size_t recs = dense_record_bytes((size_t)T, (size_t)C);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (mfma || pairs) HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
